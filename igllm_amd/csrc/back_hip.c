@@ -427,6 +427,10 @@ int igl_gemv_dev(igl_desk *desk, const igl_plane *sheet, const float *act_dev, i
       desk_fail(st, IGL_FAIL_ARGUMENT);
       return IGL_FAIL_ARGUMENT;
     }
+    if (igl_gemm_real_fits(sheet->real_type, lane_count, sheet->row_count, sheet->col_count))
+      return hip_check(st, igl_launch_gemm_real(dp->codes, sheet->real_type, act_dev, act_stride, lane_count,
+                                                out_dev, out_stride, sheet->row_count, sheet->col_count,
+                                                st->stream));
     return hip_check(st, igl_launch_gemv_real(dp->codes, sheet->real_type, act_dev, act_stride,
                                               lane_count, out_dev, out_stride, sheet->row_count,
                                               sheet->col_count, st->part_dev, st->stream));

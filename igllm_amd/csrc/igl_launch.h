@@ -77,6 +77,13 @@ hipError_t igl_launch_gemv_real(const void *rows, int real_type, const float *ac
                                 int lanes, float *out, int out_stride, int N, int K, float *part,
                                 hipStream_t stream);
 
+/* The same product on the bf16 matrix cores (bf16 and binary16 rows, five
+ * lanes and more, K a multiple of 32; arguments as igl_launch_gemv_real's,
+ * no workspace). */
+int igl_gemm_real_fits(int real_type, int lanes, int N, int K);
+hipError_t igl_launch_gemm_real(const void *rows, int real_type, const float *act, int act_stride,
+                                int lanes, float *out, int out_stride, int N, int K, hipStream_t stream);
+
 int igl_gemv_rows_per_tile(int lanes);
 int igl_gemv_chunk_cols(int lanes, int K, int lds_limit);
 size_t igl_gemv_part_floats(int lanes, int N, int K, int lds_limit);
