@@ -1,4 +1,4 @@
-// igl_gemm_real.hip - a real plane (bf16 or binary16 rows) times five lanes
+// igl_gemm_real.h - a real plane (bf16 or binary16 rows) times five lanes
 // of fp32 activations and more, gfx950 bf16 MFMA.
 //
 // C[m][n] = sum_k x[m][k] * w[n][k], the PLANE_REAL arm of back_mat_mat
@@ -36,6 +36,8 @@
 // the ks-th step of a stage, and the KS partial tiles are added in ks order at
 // the end.  The waves of a tile lie along the lanes, so no two of them split
 // the same activations.
+#pragma once
+
 #include "igl_device.h"
 #include "igl_launch.h"
 
