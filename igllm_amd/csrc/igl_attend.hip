@@ -55,11 +55,9 @@ namespace igl {
 // Positions a chunk, by the longest span a launch covers: 32 up to
 // kAttendShortSpan (the most workgroups, the shortest chain each), 64 beyond
 // (half the partials: at 16384 positions 11.4 us against 13.0 us for 32).
-// Launches of kAttendWideLanes lanes and more take 64 whatever the span: a
-// prefill pass has workgroups enough, and half the partials to fold (the
-// 2047-lane fast prefill 46 700 -> 49 300 tok/s with it on windowed spans,
-// 52 400 with it on every span; one lane keeps 32: its sliding window
-// measured 6.8 against 7.3 us with 64).
+// One lane's sliding window measured 6.8 us with 32 against 7.3 with 64.
+// Launches of kAttendWideLanes lanes and more (a prefill pass) take 64 whatever
+// the span: those of one chunk keep no partials, the others take tiles of lanes.
 constexpr int kAttendShortSpan = 8192;
 constexpr int kAttendWideLanes = 64;
 constexpr int kAttendGroup = 8;                    // query heads per key/value head
@@ -106,6 +104,7 @@ struct AttendArgs {
   float k_code_scale;
   float v_code_scale;
   float eps;
+  int lanes;                   // of the launch (tiles)
 };
 
 // Two bytes held in bits [0,8) and [16,24) of `x`, as two exact binary16.
@@ -652,262 +651,395 @@ __global__ __launch_bounds__(256) void attend_split_kernel(AttendArgs a) {
   }
 }
 
-// Wide launches (a prefill pass of kAttendWideLanes lanes or more): one
-// workgroup a lane and key/value head walks the lane's chunks of 64 positions
-// in order, each chunk's scores and blend computed as attend_split_kernel
-// computes them, and merges them into a running peak, total and blend in
-// registers (the online form of attend_fold_kernel's fold), so no partial goes
-// to memory and no fold launch follows.  The lanes give the launch its
-// workgroups, and the workgroups a CU holds hide each other's loads: three
-// at 512-dim heads (the registers capped for it, as many as their LDS
-// allows), four at 256.  Requesting the next chunk's bytes ahead in registers
-// instead held one a CU and was slower (2047 lanes, 2048 positions, 512-dim
-// heads: 955 against 667 us at two a CU, 596 at three; a 512 window of
-// 256-dim heads: 146 against 114, 109).
-template <int HEAD, int FMT, bool QVEC>
-__global__ __launch_bounds__(256, 3) void attend_rows_kernel(AttendArgs a) {
-  constexpr int C = 64;               // positions a chunk
-  constexpr int W = 4;                // waves
-  constexpr int PW = C / W;           // positions a wave scores
-  constexpr int DS = HEAD / W;        // dims a wave blends: 64 or 128
-  constexpr int S = HEAD / 32;        // k-steps of the score product
-  constexpr int QD = HEAD / 4;        // bytes of a key row one lane group reads
-  constexpr int QUADS = DS / 64;      // 64-dim groups of a wave's blend
-  constexpr int KS = C / 32;          // k-steps of the blend
-  constexpr int VP = DS + 8;          // staged value row pitch in bytes
-  constexpr int LPR = DS / 16;        // lanes that load one value row
-  constexpr int RPI = 64 / LPR;       // value rows one load instruction covers
-  constexpr int VL = C / RPI;         // value loads a lane issues
+// ---- tiles of lanes ----------------------------------------------------------
+//
+// A launch of many lanes (a prompt's pass, a block) takes tiles of 2 RB lanes:
+// their 8 query heads are the 16 RB rows of the MFMA tiles, so a key or value
+// byte is read and decoded once for all of them (a chunk workgroup decodes
+// every byte for one lane's 8, and its 16 MFMA rows hold each head's two
+// terms).  A workgroup of a wave for every 64 dims walks the chunks of 64
+// positions of the tile's span (its first lane's first position to its last
+// lane's own), or of one segment of it (blockIdx.z).  Both products are split
+// among the waves by dims: wave w takes dims 64 w .. of the scores, whose
+// partial sums the waves exchange through LDS, and the same dims of the blend.
+// So a wave holds its slice of the queries (both terms) and of the blend in
+// registers for the whole walk, and the LDS DMA brings its key and value bytes
+// into rows only it reads, the keys a chunk ahead: two barriers a chunk.
+//
+// What bounds it: a chunk's chain between the two barriers (decode, products,
+// the exchanged sums, the exponentials; 6200 cycles a chunk of 512-dim heads at
+// 32 rows, 2000 of them products on each SIMD).  At 2047 lanes, us, against one
+// workgroup a lane: 2048 positions of 512-dim heads 450 -> 118 (69 GFLOP of
+// products, two terms each: 580 TFLOP/s), a 512 window of 256-dim heads 104 -> 37;
+// 511 lanes 57 -> 22.  Four waves of 128 dims, two workgroups a CU: 129 us (a
+// chunk's chain is 8800 cycles, and the longest tile's chunks bound the launch);
+// the keys in registers instead of LDS spilled (166 us).
+//
+// Per chunk: scores S = q_lo . K^T + q_hi . K^T (the waves' sums added in wave
+// order), the rows' peak and total updated online, probabilities to LDS as two
+// binary16 terms, and blend = blend e^(old peak - peak) + (p_lo + p_hi) . V,
+// each chunk's products formed from zero.  Positions a lane does not see have
+// probability zero in its rows.
+typedef __attribute__((address_space(3))) void attend_lds_t;
+typedef __attribute__((address_space(1))) const void attend_global_t;
 
-  __shared__ half8_t qs[2][kAttendGroup][HEAD / 8];
-  __shared__ float ps[kAttendGroup][C];
-  __shared__ __attribute__((aligned(16))) float wm[W][kAttendGroup];
-  __shared__ __attribute__((aligned(16))) float wl[W][kAttendGroup];
-  __shared__ __attribute__((aligned(16))) uint8_t vs[W][C * VP];
+__device__ __forceinline__ void lds_barrier() {
+  // LDS only: the key bytes requested ahead stay in flight
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// A buffer over the rows at a uniform address: its loads take the address in
+// scalar registers and a 32-bit lane offset (as pointers, the compiler keeps
+// 64-bit lane addresses through the loop and spills).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rows(const uint8_t *rows) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(rows), 0, 0xFFFFFFFF, 0x00020000);
+}
+
+// LDS of a tile workgroup, in bytes: its waves' key rows (and then their
+// partial scores, rows of 68 floats), the probabilities' two terms (rows of 72
+// halves), a float a row, the waves' value rows.
+template <int HEAD, int RB>
+struct TileLds {
+  static constexpr int W = HEAD / 64;
+  static constexpr int KEYS = 64 * 64, SCORES = 16 * RB * 68 * 4;
+  static constexpr int KR = KEYS > SCORES ? KEYS : SCORES;
+  static constexpr int P = W * KR;
+  static constexpr int KEEP = P + 2 * 16 * RB * 72 * 2;
+  static constexpr int V = KEEP + 16 * RB * 4;
+  static constexpr int SIZE = V + 64 * HEAD;
+};
+
+template <int HEAD, int FMT, int RB, bool QVEC>
+__global__ __launch_bounds__(HEAD, 2) void attend_tile_kernel(AttendArgs a) {
+  constexpr int LT = 2 * RB;          // lanes a tile
+  constexpr int ROWS = 16 * RB;       // (lane, head) rows
+  constexpr int C = 64;               // positions a chunk
+  constexpr int W = HEAD / 64;        // waves: a thread a dim
+  constexpr int DS = 64;              // dims a wave holds
+  constexpr int S = DS / 32;          // k-steps of its scores
+  constexpr int QD = DS / 4;          // dims (and key bytes a position) one lane group reads
+  constexpr int LPR = DS / 16;        // 16-byte chunks of a staged value row
+  constexpr int RPI = 64 / LPR;       // value rows one DMA instruction covers
+  constexpr int VL = C / RPI;         // DMA instructions of a chunk's values
+  constexpr int RP = C + 4;           // score row pitch in floats
+  constexpr int PP = C + 8;           // probability row pitch in halves
+  constexpr int TPR = HEAD / ROWS < 16 ? HEAD / ROWS : 16;  // threads a row in the softmax
+  constexpr int PPT = C / TPR;        // positions a thread
+
+  // one array, laid out by hand: between arrays the compiler would wait for
+  // the DMA into one before any read of another
+  using F = TileLds<HEAD, RB>;
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  _Float16 *ph = reinterpret_cast<_Float16 *>(lds + F::P), *pl = ph + ROWS * PP;
+  float *keep_s = reinterpret_cast<float *>(lds + F::KEEP);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4;
   const int n = lane & 15;
   const int kv = blockIdx.y;
   const int head0 = kv * kAttendGroup;
-  // the last lanes, with the most chunks, first: the workgroups are handed
-  // out in grid order, and the long ones would otherwise start last
-  const int lane_id = (int)gridDim.z - 1 - (int)blockIdx.z;
-  const int pos0 = a.place_dev ? *a.place_dev : a.place0;
-  const int pos = pos0 + lane_id;
-  const int span = a.window > 0 ? min(pos + 1, a.window) : pos + 1;
-  const int place_start = pos - span + 1;
-  const int blocks = (span + C - 1) / C;
   const size_t kv_off = (size_t)kv * HEAD;
-  const int ring0 = place_start % a.cache_span;
+  // Longest tiles first, as a CU frees.  Where two workgroups share a CU and
+  // all fit at once (256-dim heads), the second half starts with the shortest,
+  // so a causal launch's long tiles each meet a short one on their CU.
+  const int tiles = gridDim.x, half = W == 4 && tiles <= 512 ? (tiles + 1) / 2 : tiles;
+  const int tile = (int)blockIdx.x < half ? tiles - 1 - (int)blockIdx.x : (int)blockIdx.x - half;
+  const int l0 = tile * LT;
+  const int ln = min(LT, a.lanes - l0);
+  const int pos0 = __builtin_amdgcn_readfirstlane(a.place_dev ? *a.place_dev : a.place0) + l0;
+  const int start = a.window > 0 ? max(0, pos0 + 1 - a.window) : 0;
+  const int span = pos0 + ln - start;  // of the tile
+  const int chunks = (span + C - 1) / C;
+  const int per = (chunks + (int)gridDim.z - 1) / (int)gridDim.z;
+  const int seg = blockIdx.z;
+  const int c_first = seg * per, c_end = min(chunks, c_first + per);
+  const bool split = gridDim.z > 1;
+
+  // the softmax's row of this thread, its lane's visible positions (relative
+  // to start) and its running peak and total
+  const int row = min(tid / TPR, ROWS - 1);
+  const int li = min(row / kAttendGroup, ln - 1);
+  const int see_end = pos0 + li - start;  // inclusive
+  const int see_first = a.window > 0 ? max(0, pos0 + li + 1 - a.window) - start : 0;
+  float run_m = -INFINITY, run_l = 0.0f;
+
+  const int ring0 = start % a.cache_span;
+  // t < span < 2 cache_span (the host takes this form past 64 visible positions)
   auto ring_slot = [&](int t) {
-    const int slot = ring0 + t;
+    int slot = ring0 + t;
+    slot = slot >= a.cache_span ? slot - a.cache_span : slot;
     return slot >= a.cache_span ? slot - a.cache_span : slot;
   };
-  // key row of chunk b: position b C + wave PW + n, bytes QD g .. QD g + QD - 1;
-  // value rows: lane / LPR + RPI i, dims wave DS + 16 (lane % LPR) .. + 15
-  auto load_keys = [&](int b, uint4_t (&kr)[QD / 16]) {
-    const int t = min(b * C + wave * PW + n, span - 1);
-    const uint4_t *row =
-        reinterpret_cast<const uint4_t *>(a.key_store + (size_t)ring_slot(t) * a.kv_width + kv_off + QD * g);
+  // A whole chunk in consecutive slots (nearly all are) is read at lane
+  // offsets from one uniform address; else each row finds its own slot.
+  // Key row p holds its 16-byte chunk ch at chunk ch ^ (p / 4) % 4, so the 16
+  // rows a score read spans lie in distinct banks.
+  uint8_t *kw = lds + F::KR * wave;
+  const int k_row = lane / LPR;
+  const int k_chunk = 16 * ((lane % 4) ^ (lane >> 4));
+  const uint32_t k_lane = (uint32_t)(k_row * a.kv_width + k_chunk);
+  auto load_keys = [&](int c) {
+    const int slot0 = ring_slot(c * C);
+    const uint8_t *keys = a.key_store + kv_off + wave * DS;
+    if (c * C + C <= span && slot0 + C <= a.cache_span) {
+      const auto src = uniform_rows(keys + (size_t)slot0 * a.kv_width);
 #pragma unroll
-    for (int q = 0; q < QD / 16; ++q) kr[q] = __builtin_nontemporal_load(row + q);
-  };
-  auto load_values = [&](int b, uint4_t (&vr)[VL]) {
-#pragma unroll
-    for (int i = 0; i < VL; ++i) {
-      const int t = min(b * C + lane / LPR + RPI * i, span - 1);
-      vr[i] = __builtin_nontemporal_load(reinterpret_cast<const uint4_t *>(
-          a.value_store + (size_t)ring_slot(t) * a.kv_width + kv_off + wave * DS + 16 * (lane % LPR)));
-    }
-  };
-
-  // ---- the query, once: x = hi + lo in binary16
-  constexpr int kQItems = kAttendGroup * HEAD / 8 / 256;
-  {
-    float qf[kQItems][8];
-    const float *qb = a.query + (size_t)lane_id * a.q_stride + (size_t)head0 * HEAD;
-#pragma unroll
-    for (int i = 0; i < kQItems; ++i) {
-      const float *q = qb + 8 * (tid + 256 * i);
-      if (QVEC) {
-        const float4_t u = *reinterpret_cast<const float4_t *>(q);
-        const float4_t v = *reinterpret_cast<const float4_t *>(q + 4);
-        qf[i][0] = u.x; qf[i][1] = u.y; qf[i][2] = u.z; qf[i][3] = u.w;
-        qf[i][4] = v.x; qf[i][5] = v.y; qf[i][6] = v.z; qf[i][7] = v.w;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) qf[i][e] = q[e];
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < kQItems; ++i) {
-      half8_t hi8, lo8;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const _Float16 hi = (_Float16)qf[i][e];
-        hi8[e] = hi;
-        lo8[e] = (_Float16)(qf[i][e] - (float)hi);
-      }
-      const int item = tid + 256 * i;
-      qs[0][item / (HEAD / 8)][item % (HEAD / 8)] = hi8;
-      qs[1][item / (HEAD / 8)][item % (HEAD / 8)] = lo8;
-    }
-  }
-
-  // running peak, total and blend of heads 4g + r (lanes g < 2), dims
-  // wave DS + 64 qd + 4 n + t
-  float run_m[4], run_l[4];
-  float4_t run_o[4 * QUADS];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    run_m[r] = -INFINITY;
-    run_l[r] = 0.0f;
-  }
-#pragma unroll
-  for (int t = 0; t < 4 * QUADS; ++t) run_o[t] = float4_t{0, 0, 0, 0};
-
-  uint4_t kr[QD / 16], vr[VL];
-  const int hh = n & 7;
-  for (int b = 0; b < blocks; ++b) {
-    __syncthreads();  // the query in LDS; the chunk before done with ps, wm, wl, vs
-    const int c0 = b * C;
-    // requested after the barrier: before it, 709 against 667 us (2047 lanes,
-    // 2048 positions, 512-dim heads)
-    load_keys(b, kr);
-    load_values(b, vr);
-    // scores of the wave's PW positions for the 8 heads, all dims
-    float sc[4], m_w[4];
-    {
-      float4_t sacc = float4_t{0, 0, 0, 0};
-#pragma unroll
-      for (int s = 0; s < S; ++s) {
-        const half8_t qa = qs[n >> 3][n & 7][QD * g / 8 + s];
-        const uint4_t w = kr[s >> 1];
-        const half8_t kb = (s & 1) ? decode8<FMT>(w[2], w[3]) : decode8<FMT>(w[0], w[1]);
-        sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa, kb, sacc, 0, 0, 0);
-      }
-      const bool valid = c0 + wave * PW + n < span;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float v = xsum32(sacc[r]);
-        sc[r] = valid ? v * a.key_scale : -INFINITY;
-        m_w[r] = row16_max(sc[r]);
-      }
-    }
-    {
-      float l_w[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float p = m_w[r] != -INFINITY && sc[r] != -INFINITY ? __expf(sc[r] - m_w[r]) : 0.0f;
-        l_w[r] = row16_sum(p);
-        if (g < 2) ps[4 * g + r][wave * PW + n] = p;
-      }
-      if (g < 2 && n == 0) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          wm[wave][4 * g + r] = m_w[r];
-          wl[wave][4 * g + r] = l_w[r];
-        }
-      }
-    }
-    {
-      uint8_t *vw = vs[wave];
+      for (int i = 0; i < VL; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (attend_lds_t *)(kw + 1024 * i), 16, k_lane,
+                                                 RPI * i * a.kv_width, 0, 0);
+    } else {
 #pragma unroll
       for (int i = 0; i < VL; ++i) {
-        uint2_t *dst = reinterpret_cast<uint2_t *>(vw + (lane / LPR + RPI * i) * VP + 16 * (lane % LPR));
-        dst[0] = uint2_t{vr[i][0], vr[i][1]};
-        dst[1] = uint2_t{vr[i][2], vr[i][3]};
+        const int t = min(c * C + RPI * i + k_row, span - 1);
+        __builtin_amdgcn_global_load_lds(
+            (attend_global_t *)(keys + (size_t)ring_slot(t) * a.kv_width + k_chunk),
+            (attend_lds_t *)(kw + 1024 * i), 16, 0, 0);
       }
     }
-    __syncthreads();
-    // blend of the wave's dims over the chunk, against the chunk's peak M
-    float M = wm[0][hh];
+  };
+  // Value row p goes to row slot (p & ~3) + (p + p / 8) % 4: a blend read takes
+  // 64 bytes of rows p, p + 8, p + 16 and p + 24, which so lie in four distinct
+  // quarters of the banks.  Instruction i fills slots RPI i + lane / LPR; v_row
+  // is the lane's row in an even and an odd one.
+  uint8_t *vw = lds + F::V + C * DS * wave;
+  int v_row[2];
+  uint32_t v_lane[2];
 #pragma unroll
-    for (int w = 1; w < W; ++w) M = fmaxf(M, wm[w][hh]);
-    float4_t o[4 * QUADS];
+  for (int o = 0; o < 2; ++o) {
+    v_row[o] = ((lane / LPR) & ~3) | ((lane / LPR - 2 * o - (lane >> 5)) & 3);
+    v_lane[o] = (uint32_t)(v_row[o] * a.kv_width + 16 * (lane % LPR));
+  }
+  auto load_values = [&](int c) {
+    const int slot0 = ring_slot(c * C);
+    const uint8_t *values = a.value_store + kv_off + wave * DS;
+    if (c * C + C <= span && slot0 + C <= a.cache_span) {
+      const auto src = uniform_rows(values + (size_t)slot0 * a.kv_width);
 #pragma unroll
-    for (int t = 0; t < 4 * QUADS; ++t) o[t] = float4_t{0, 0, 0, 0};
-    const uint8_t *vw = vs[wave];
+      for (int i = 0; i < VL; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (attend_lds_t *)(vw + 1024 * i), 16,
+                                                 v_lane[i & 1], RPI * i * a.kv_width, 0, 0);
+    } else {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int p0 = 32 * ks + 8 * g;
-      const float mw = wm[p0 / PW][hh];
-      const float f = mw != -INFINITY ? __expf(mw - M) : 0.0f;
-      half8_t pa;
-      {
-        const float *src = &ps[hh][p0];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float v = src[e] * f;
-          const _Float16 hi = (_Float16)v;
-          pa[e] = n >= 8 ? (_Float16)(v - (float)hi) : hi;
-        }
-      }
-#pragma unroll
-      for (int qd = 0; qd < QUADS; ++qd) {
-        uint32_t dw[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          dw[e] = *reinterpret_cast<const uint32_t *>(vw + (p0 + e) * VP + 64 * qd + 4 * n);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          uint32_t w[4];
-          const uint32_t sel = 0x0C000C00u | ((uint32_t)(4 + t) << 16) | (uint32_t)t;
-#pragma unroll
-          for (int pr = 0; pr < 4; ++pr)
-            w[pr] = decode_pair<FMT>(__builtin_amdgcn_perm(dw[2 * pr + 1], dw[2 * pr], sel));
-          o[4 * qd + t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa, __builtin_bit_cast(half8_t, w),
-                                                                 o[4 * qd + t], 0, 0, 0);
-        }
+      for (int i = 0; i < VL; ++i) {
+        const int t = min(c * C + RPI * i + v_row[i & 1], span - 1);
+        __builtin_amdgcn_global_load_lds(
+            (attend_global_t *)(values + (size_t)ring_slot(t) * a.kv_width + 16 * (lane % LPR)),
+            (attend_lds_t *)(vw + 1024 * i), 16, 0, 0);
       }
     }
+  };
+  // the lane's blend reads of its eight rows p0 .. p0 + 7 (p0 = 32 ks + 8 g)
+  const uint8_t *v_read[4];
 #pragma unroll
-    for (int t = 0; t < 4 * QUADS; ++t)
+  for (int e = 0; e < 4; ++e) v_read[e] = vw + 512 * g + 64 * ((e + g) & 3) + 4 * n;
+  if (c_first < c_end) load_keys(c_first);
+
+  // the wave's slice of the queries, x = hi + lo: row 16 rb + n is lane 2 rb +
+  // n / 8, head n % 8; k-step s of lane group g is dims QD g + 8 s .. + 7
+  half8_t qh[RB][S], ql[RB][S];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[t][r] = xsum32(o[t][r]);
-    // merge the chunk (peak Mh, total L, blend o) into the running state
-    if (g < 2) {
-      float4_t pk[W], tl[W];
+  for (int rb = 0; rb < RB; ++rb) {
+    const int lq = l0 + min(2 * rb + (n >> 3), ln - 1);
+    const float *q = a.query + (size_t)lq * a.q_stride + (size_t)(head0 + (n & 7)) * HEAD + wave * DS + QD * g;
 #pragma unroll
-      for (int w = 0; w < W; ++w) {
-        pk[w] = *reinterpret_cast<const float4_t *>(&wm[w][4 * g]);
-        tl[w] = *reinterpret_cast<const float4_t *>(&wl[w][4 * g]);
+    for (int s = 0; s < S; ++s) {
+      float x[8];
+      if (QVEC) {
+        const float4_t u = *reinterpret_cast<const float4_t *>(q + 8 * s);
+        const float4_t v = *reinterpret_cast<const float4_t *>(q + 8 * s + 4);
+        x[0] = u.x; x[1] = u.y; x[2] = u.z; x[3] = u.w;
+        x[4] = v.x; x[5] = v.y; x[6] = v.z; x[7] = v.w;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = q[8 * s + e];
       }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float Mh = pk[0][r];
-#pragma unroll
-        for (int w = 1; w < W; ++w) Mh = fmaxf(Mh, pk[w][r]);
-        float L = 0.0f;
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-          const float e = pk[w][r] != -INFINITY ? __expf(pk[w][r] - Mh) : 0.0f;
-          L += tl[w][r] * e;
-        }
-        const float Mn = fmaxf(run_m[r], Mh);
-        const float keep = run_m[r] != -INFINITY ? __expf(run_m[r] - Mn) : 0.0f;
-        const float take = Mh != -INFINITY ? __expf(Mh - Mn) : 0.0f;
-        run_l[r] = run_l[r] * keep + L * take;
-#pragma unroll
-        for (int t = 0; t < 4 * QUADS; ++t) run_o[t][r] = run_o[t][r] * keep + o[t][r] * take;
-        run_m[r] = Mn;
+      for (int e = 0; e < 8; ++e) {
+        const _Float16 hi = (_Float16)x[e];
+        qh[rb][s][e] = hi;
+        ql[rb][s][e] = (_Float16)(x[e] - (float)hi);
       }
     }
   }
-  if (g >= 2) return;
+
+  // the blend: rows 16 rb + 4 g + r, dims wave DS + 4 n + t
+  float4_t out[RB][4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int h = 4 * g + r;
-    const float mul = run_l[r] > 0.0f ? a.value_scale * (1.0f / run_l[r]) : 0.0f;
-    float *dst = a.final_out + (size_t)lane_id * a.q_stride + (size_t)(head0 + h) * HEAD + wave * DS + 4 * n;
+  for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-    for (int qd = 0; qd < QUADS; ++qd)
-      *reinterpret_cast<float4_t *>(dst + 64 * qd) = float4_t{run_o[4 * qd][r] * mul, run_o[4 * qd + 1][r] * mul,
-                                                              run_o[4 * qd + 2][r] * mul, run_o[4 * qd + 3][r] * mul};
+    for (int t = 0; t < 4; ++t) out[rb][t] = float4_t{0, 0, 0, 0};
+
+  for (int c = c_first; c < c_end; ++c) {
+    asm volatile("" ::: "memory");
+    load_values(c);  // the chunk before's reads of these rows have been multiplied
+    __builtin_amdgcn_s_waitcnt(0xF70 | VL);  // the keys, requested before, have landed
+    asm volatile("" ::: "memory");
+    // scores over the wave's dims
+    float4_t sc[RB][4];
+#pragma unroll
+    for (int pb = 0; pb < 4; ++pb) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) sc[rb][pb] = float4_t{0, 0, 0, 0};
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        const uint4_t w = *reinterpret_cast<const uint4_t *>(kw + (16 * pb + n) * DS + 16 * (g ^ (n >> 2)));
+        const half8_t kb = (s & 1) ? decode8<FMT>(w[2], w[3]) : decode8<FMT>(w[0], w[1]);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          sc[rb][pb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ql[rb][s], kb, sc[rb][pb], 0, 0, 0);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          sc[rb][pb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh[rb][s], kb, sc[rb][pb], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int pb = 0; pb < 4; ++pb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) reinterpret_cast<float *>(kw)[(16 * rb + 4 * g + r) * RP + 16 * pb + n] = sc[rb][pb][r];
+    lds_barrier();
+    // the row's scores of this thread, its peak and total, its probabilities
+    if (ROWS * TPR == HEAD || tid < ROWS * TPR) {
+      const int p0 = PPT * (tid % TPR);
+      float v[PPT];
+#pragma unroll
+      for (int e = 0; e < PPT; e += 4) {
+        float4_t x[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) x[w] = reinterpret_cast<const float4_t *>(lds + F::KR * w)[(row * RP + p0 + e) / 4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+          for (int w = W / 2; w > 0; w >>= 1)
+#pragma unroll
+            for (int j = 0; j < w; ++j) x[j][i] += x[j + w][i];
+          v[e + i] = x[0][i] * a.key_scale;
+        }
+      }
+      // uniform in a wave: some of its rows do not see all of the chunk
+      const int t0 = c * C;
+      if (t0 < see_first || t0 + C - 1 > see_end) {
+#pragma unroll
+        for (int e = 0; e < PPT; ++e) {
+          const int t = t0 + p0 + e;
+          if (t < see_first || t > see_end) v[e] = -INFINITY;
+        }
+      }
+      float peak = v[0];
+#pragma unroll
+      for (int e = 1; e < PPT; ++e) peak = fmaxf(peak, v[e]);
+      peak = fmaxf(peak, dpp_move<0xB1>(peak));
+      peak = fmaxf(peak, dpp_move<0x4E>(peak));
+      if (TPR >= 8) peak = fmaxf(peak, dpp_move<0x141>(peak));
+      if (TPR >= 16) peak = fmaxf(peak, dpp_move<0x140>(peak));
+      const float m = fmaxf(run_m, peak);
+      const float keep = run_m != -INFINITY ? __expf(run_m - m) : 0.0f;
+      float total = 0.0f;
+      _Float16 hi[PPT], lo[PPT];
+#pragma unroll
+      for (int e = 0; e < PPT; ++e) {
+        const float p = v[e] != -INFINITY ? __expf(v[e] - m) : 0.0f;
+        total += p;
+        hi[e] = (_Float16)p;
+        lo[e] = (_Float16)(p - (float)hi[e]);
+      }
+      total += dpp_move<0xB1>(total);
+      total += dpp_move<0x4E>(total);
+      if (TPR >= 8) total += dpp_move<0x141>(total);
+      if (TPR >= 16) total += dpp_move<0x140>(total);
+      run_l = run_l * keep + total;
+      run_m = m;
+      __builtin_memcpy(__builtin_assume_aligned(&ph[row * PP + p0], 8), hi, sizeof(hi));
+      __builtin_memcpy(__builtin_assume_aligned(&pl[row * PP + p0], 8), lo, sizeof(lo));
+      if (tid % TPR == 0) keep_s[row] = keep;
+    }
+    // the wave's values have landed: their reads go out before the barrier
+    __builtin_amdgcn_s_waitcnt(0xF70);
+    asm volatile("" ::: "memory");
+    uint32_t dw[C / 32][8];
+#pragma unroll
+    for (int ks = 0; ks < C / 32; ++ks)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        dw[ks][e] = *reinterpret_cast<const uint32_t *>(v_read[e & 3] + 2048 * ks + 256 * (e >> 2));
+    lds_barrier();
+    if (c + 1 < c_end) load_keys(c + 1);  // every wave has read the scores that lay there
+    // the blend over the wave's dims
+    float4_t o[RB][4];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) o[rb][t] = float4_t{0, 0, 0, 0};
+#pragma unroll
+    for (int ks = 0; ks < C / 32; ++ks) {
+      half8_t pa[RB][2];
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        pa[rb][0] = *reinterpret_cast<const half8_t *>(&ph[(16 * rb + n) * PP + 32 * ks + 8 * g]);
+        pa[rb][1] = *reinterpret_cast<const half8_t *>(&pl[(16 * rb + n) * PP + 32 * ks + 8 * g]);
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        uint32_t w[4];
+        const uint32_t sel = 0x0C000C00u | ((uint32_t)(4 + t) << 16) | (uint32_t)t;
+#pragma unroll
+        for (int pr = 0; pr < 4; ++pr)
+          w[pr] = decode_pair<FMT>(__builtin_amdgcn_perm(dw[ks][2 * pr + 1], dw[ks][2 * pr], sel));
+        const half8_t vb = __builtin_bit_cast(half8_t, w);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          o[rb][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[rb][1], vb, o[rb][t], 0, 0, 0);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          o[rb][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[rb][0], vb, o[rb][t], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      const float4_t keep = *reinterpret_cast<const float4_t *>(&keep_s[16 * rb + 4 * g]);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[rb][t][r] = __builtin_fmaf(out[rb][t][r], keep[r], o[rb][t][r]);
+    }
   }
+
+  // the rows' totals to every wave; with segments the partial, else the blend
+  lds_barrier();
+  if (tid % TPR == 0 && tid < ROWS * TPR) {
+    keep_s[row] = run_l;
+    if (split && row / kAttendGroup < ln) {
+      const size_t at = ((size_t)(l0 + row / kAttendGroup) * gridDim.z + seg) * a.head_count + head0 + (row & 7);
+      a.part_peak[at] = run_m;
+      a.part_total[at] = run_l;
+    }
+  }
+  lds_barrier();
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int m = 16 * rb + 4 * g + r;
+      const int l = m / kAttendGroup, h = head0 + (m & 7);
+      if (l >= ln) continue;
+      const float total = keep_s[m];
+      const float mul = split ? a.value_scale : total > 0.0f ? a.value_scale * (1.0f / total) : 0.0f;
+      float *dst = (split ? a.part_out + (((size_t)(l0 + l) * gridDim.z + seg) * a.head_count + h) * HEAD
+                          : a.final_out + (size_t)(l0 + l) * a.q_stride + (size_t)h * HEAD) + wave * DS + 4 * n;
+      const float4_t o4 = {out[rb][0][r] * mul, out[rb][1][r] * mul, out[rb][2][r] * mul, out[rb][3][r] * mul};
+      if (QVEC || split) {
+        *reinterpret_cast<float4_t *>(dst) = o4;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dst[e] = o4[e];
+      }
+    }
 }
 
 // Folds chunk partials in one memory round trip.  A workgroup per (head, lane,
@@ -936,7 +1068,8 @@ __global__ __launch_bounds__(256) void attend_fold_kernel(const float *part_out_
   // extra: the block's new positions up to the lane's own have a partial of
   // their own, after the chunks of the positions before the block
   const int fresh = extra ? lane_id + 1 : 0;
-  const int chunks = (span - fresh + chunk - 1) / chunk + (extra ? 1 : 0);
+  // chunk 0: every lane fills its slots, those of no position with a zero blend
+  const int chunks = chunk ? (span - fresh + chunk - 1) / chunk + (extra ? 1 : 0) : chunk_slots;
   const size_t base = (size_t)lane_id * chunk_slots;
   const size_t step = (size_t)head_count * head_size;
   const float *pout = part_out_all + base * step + (size_t)h * head_size + blockIdx.z * DIMS + d;
@@ -1010,6 +1143,63 @@ static int attend_blocks(int place0, int window, int lanes) {
   return (attend_max_span(place0, window, lanes) + chunk - 1) / chunk;
 }
 
+// Which launches take tiles of lanes (attend_tile_kernel), and their shape.
+//
+// Spans past 64 positions (up to there one chunk workgroup a lane writes the
+// blend), and
+//   * from 64 lanes: always;
+//   * below: two lanes and more of 512-dim heads; of 256-dim heads where the
+//     chunk form would take 512 workgroups and more.  Replayed, us, chunk
+//     workgroups and fold -> tiles: 512 dims, 2 lanes at 300 positions 9.9 -> 8.6
+//     (16000: 22.5 -> 15.5), 16 lanes 11.2 -> 9.3, 63 lanes 23.3 -> 14.4, 32
+//     lanes at 16000 216 -> 40; 256 dims, 63 lanes of a 512 window 15.8 -> 11.9, 5
+//     lanes at 16000 26.7 -> 14.9, but 4 lanes of the window 7.7 against 7.9, 16
+//     lanes 8.5 against 8.9, 2 lanes at 16000 (502 chunk workgroups) 12.8
+//     against 13.2.
+// Tiles of two lanes up to 512 of them, of four beyond (1000 lanes of 512 dims
+// 43.2 us in twos, 49.3 in fours; 2047 lanes 153 against 118).
+//
+// Few tiles are cut into segments of their chunks, folded by a second launch:
+// as many as fill 256 workgroups, 512 (512 dims) or 1024 (256 dims) where a
+// segment would still be more than eight chunks long, 64 at most.  100 lanes at
+// 2000 positions, 256 dims: unsplit 55.7 us, five segments 22; 300 lanes of a
+// 512 window: unsplit 19.0, two 22.5; 32 lanes at 16000, 512 dims: 16 segments
+// 44.2, 32 40.4, 64 45.6.  The partials stay within what the same call's chunk
+// form takes below 64 lanes; from there within what 48 lanes' chunk form would
+// take (the engine's workspace holds 63 lanes') and IGL_ATTEND_FIXED_FLOATS.
+struct TilePlan {
+  int rb;        // lanes a tile / 2; 0: not this form
+  int segments;
+};
+
+static TilePlan attend_tile_plan(int place0, int window, int lanes, int head_count, int head_size) {
+  const TilePlan none = {0, 1};
+  if (lanes < 2) return none;
+  const int span = attend_max_span(place0, window, lanes);
+  const int kv_count = head_count / kAttendGroup;
+  const bool wide = lanes >= kAttendWideLanes;
+  const long blocks = (span + (span <= kAttendShortSpan ? 31 : 63)) / (span <= kAttendShortSpan ? 32 : 64);
+  if (span <= 64) return none;
+  if (!wide && head_size == 256 && (long)lanes * kv_count * blocks < 512) return none;
+  const int rb = (long)((lanes + 1) / 2) * kv_count <= 512 ? 1 : 2;
+  const long tiles = (long)((lanes + 2 * rb - 1) / (2 * rb)) * kv_count;
+  const long chunks = (span + 2 * rb - 1 + 63) / 64;  // of a tile, at most
+  long s = 256 / tiles;
+  if (s < 1) s = 1;
+  if (chunks > 8 * s) s = (head_size == 256 ? 1024 : 512) / tiles;
+  if (wide) {
+    const long fixed = (long)IGL_ATTEND_FIXED_FLOATS / ((long)lanes * head_count * (head_size + 2));
+    if (s > 48 * blocks / lanes) s = 48 * blocks / lanes;
+    if (s > fixed) s = fixed;
+  }
+  if (s > 64) s = 64;
+  if (s > blocks) s = blocks;
+  if (s > chunks) s = chunks;
+  if (s < 1) s = 1;
+  const long per = (chunks + s - 1) / s;
+  return TilePlan{rb, (int)((chunks + per - 1) / per)};
+}
+
 template <int HEAD, int FMT, int C>
 static void attend_launch(const AttendArgs &a, dim3 grid, bool qvec, hipStream_t stream) {
   if (qvec)
@@ -1018,12 +1208,29 @@ static void attend_launch(const AttendArgs &a, dim3 grid, bool qvec, hipStream_t
     hipLaunchKernelGGL((attend_split_kernel<HEAD, FMT, C, false, false>), grid, dim3(256), 0, stream, a);
 }
 
+template <int HEAD, int FMT, int RB, bool QVEC>
+static hipError_t attend_launch_tiles(const AttendArgs &a, int kv_count, int segments, hipStream_t stream) {
+  constexpr int size = TileLds<HEAD, RB>::SIZE;
+  static bool granted = false;  // the dynamic LDS a kernel asks for is granted once
+  if (!granted) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&attend_tile_kernel<HEAD, FMT, RB, QVEC>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, size);
+    if (e != hipSuccess) return e;
+    granted = true;
+  }
+  const dim3 grid((a.lanes + 2 * RB - 1) / (2 * RB), kv_count, segments);
+  hipLaunchKernelGGL((attend_tile_kernel<HEAD, FMT, RB, QVEC>), grid, dim3(HEAD), (size_t)size, stream, a);
+  return hipGetLastError();
+}
+
 template <int HEAD, int FMT>
-static void attend_launch_rows(const AttendArgs &a, dim3 grid, bool qvec, hipStream_t stream) {
-  if (qvec)
-    hipLaunchKernelGGL((attend_rows_kernel<HEAD, FMT, true>), grid, dim3(256), 0, stream, a);
-  else
-    hipLaunchKernelGGL((attend_rows_kernel<HEAD, FMT, false>), grid, dim3(256), 0, stream, a);
+static hipError_t attend_launch_tile(const AttendArgs &a, const TilePlan &p, int kv_count, bool qvec,
+                                     hipStream_t stream) {
+  if (p.rb == 1)
+    return qvec ? attend_launch_tiles<HEAD, FMT, 1, true>(a, kv_count, p.segments, stream)
+                : attend_launch_tiles<HEAD, FMT, 1, false>(a, kv_count, p.segments, stream);
+  return qvec ? attend_launch_tiles<HEAD, FMT, 2, true>(a, kv_count, p.segments, stream)
+              : attend_launch_tiles<HEAD, FMT, 2, false>(a, kv_count, p.segments, stream);
 }
 
 template <int HEAD, int FMT>
@@ -1063,6 +1270,7 @@ extern "C" hipError_t igl_launch_attend(const uint8_t *key_store, const uint8_t 
   a.place0 = place0;
   a.place_dev = place_dev;
   a.window = window;
+  a.lanes = lanes;
   a.chunks = chunks;
   a.final_out = chunks == 1 ? blend_out : nullptr;
   a.q_stride = q_stride;
@@ -1081,21 +1289,22 @@ extern "C" hipError_t igl_launch_attend(const uint8_t *key_store, const uint8_t 
   a.k_code_scale = a.v_code_scale = a.eps = 0.0f;
   dim3 grid(chunks, kv_count, lanes);
   const bool qvec = (((uintptr_t)query) & 15u) == 0 && (q_stride & 3) == 0;
-  if (lanes >= kAttendWideLanes && chunks > 1) {
-    // a prefill pass: one workgroup a lane walks its chunks, no partials
+  const TilePlan plan = attend_tile_plan(place0, window, lanes, head_count, head_size);
+  if (plan.rb) {
     a.final_out = blend_out;
-    const dim3 rows(1, kv_count, lanes);
+    a.part_peak = work + (size_t)lanes * plan.segments * head_count * head_size;
+    a.part_total = a.part_peak + (size_t)lanes * plan.segments * head_count;
+    hipError_t e = hipErrorInvalidValue;
     if (head_size == 256 && fmt == 0)
-      attend_launch_rows<256, 0>(a, rows, qvec, stream);
+      e = attend_launch_tile<256, 0>(a, plan, kv_count, qvec, stream);
     else if (head_size == 256 && fmt == 1)
-      attend_launch_rows<256, 1>(a, rows, qvec, stream);
+      e = attend_launch_tile<256, 1>(a, plan, kv_count, qvec, stream);
     else if (head_size == 512 && fmt == 0)
-      attend_launch_rows<512, 0>(a, rows, qvec, stream);
+      e = attend_launch_tile<512, 0>(a, plan, kv_count, qvec, stream);
     else if (head_size == 512 && fmt == 1)
-      attend_launch_rows<512, 1>(a, rows, qvec, stream);
-    else
-      return hipErrorInvalidValue;
-    return hipGetLastError();
+      e = attend_launch_tile<512, 1>(a, plan, kv_count, qvec, stream);
+    if (e != hipSuccess || plan.segments == 1) return e;
+    return attend_fold(a, plan.segments, 0, place0, place_dev, window, lanes, head_size, blend_out, stream);
   }
   if (head_size == 256 && fmt == 0)
     attend_launch_chunk<256, 0>(a, grid, chunk, qvec, stream);
@@ -1196,6 +1405,7 @@ extern "C" hipError_t igl_launch_attend_prep(const uint8_t *key_store, const uin
   a.place0 = place_bound;
   a.place_dev = place_dev;
   a.window = window;
+  a.lanes = lanes;
   a.chunks = chunks;
   a.final_out = chunks == 1 && !extra ? blend_out : nullptr;
   a.q_stride = lanes > 1 ? q_stride : kAttendGroup * head_size;
@@ -1247,9 +1457,12 @@ extern "C" size_t igl_attend_prep_work_floats(int place_bound, int window, int h
 extern "C" size_t igl_attend_work_floats(int place0, int window, int lanes, int head_count,
                                          int head_size) {
   const size_t blocks = (size_t)attend_blocks(place0, window, lanes);
-  // a wide launch of more than one chunk merges its chunks in registers
-  // (attend_rows_kernel): no partials
-  if (lanes >= kAttendWideLanes && blocks > 1) return 0;
+  // from kAttendWideLanes lanes, more than one chunk: the tiles' segments, or
+  // no partials (below, the tiles' segments take no more than the chunks)
+  if (lanes >= kAttendWideLanes && blocks > 1) {
+    const int segments = attend_tile_plan(place0, window, lanes, head_count, head_size).segments;
+    return segments == 1 ? 0 : (size_t)lanes * segments * (size_t)head_count * ((size_t)head_size + 2);
+  }
   return (size_t)lanes * blocks * (size_t)head_count * ((size_t)head_size + 2);
 }
 
@@ -1258,9 +1471,8 @@ extern "C" size_t igl_attend_work_floats(int place0, int window, int lanes, int 
 // count is not monotonic in the span: chunks are 32 positions up to
 // kAttendShortSpan and 64 beyond, so a span just under kAttendShortSpan has
 // more chunks than one just over it.  The largest count of each regime is
-// taken.  Launches of kAttendWideLanes lanes and more keep no partials (one
-// chunk: the blend written directly; more: merged in registers), so the most
-// lanes that keep partials is kAttendWideLanes - 1.
+// taken.  A launch of kAttendWideLanes lanes and more keeps fewer partials than
+// kAttendWideLanes - 1 lanes over the same span (attend_tile_plan).
 extern "C" size_t igl_attend_work_floats_limit(int span_limit, int lanes, int head_count,
                                                int head_size) {
   if (span_limit < 1 || lanes < 1) return 0;
