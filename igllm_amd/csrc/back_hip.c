@@ -445,6 +445,12 @@ int igl_gemv_dev(igl_desk *desk, const igl_plane *sheet, const float *act_dev, i
                                                out_stride, sheet->row_count, sheet->col_count,
                                                st->part_dev, st->stream));
   }
+  if (igl_gemm_few_fits(lane_count, sheet->row_count, sheet->col_count) &&
+      ((uintptr_t)act_dev & 15u) == 0 && (act_stride & 3) == 0)
+    return hip_check(st, igl_launch_gemm_few((const uint8_t *)dp->codes, (long long)sheet->row_stride, dp->gains,
+                                             sheet->group_count, igl_plane_group_shift(sheet), act_dev, act_stride,
+                                             lane_count, out_dev, out_stride, sheet->row_count, sheet->col_count,
+                                             st->stream));
   for (done = 0; done < lane_count; done += IGL_GEMV_Q4_LANES) {
     int lanes = lane_count - done < IGL_GEMV_Q4_LANES ? lane_count - done : IGL_GEMV_Q4_LANES;
     hipError_t e = igl_launch_gemv_q4(

@@ -853,5 +853,7 @@ extern "C" hipError_t igl_launch_gemm_q4(const void *act, int act_bf16, int act_
   return hipGetLastError();
 }
 
-// The real planes' product (igl_launch_gemm_real), its own kernels and forms.
+// The real planes' product and the few-lane product, each its own kernels and
+// forms.
 #include "igl_gemm_real.h"
+#include "igl_gemm_few.h"

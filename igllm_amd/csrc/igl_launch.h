@@ -84,6 +84,14 @@ int igl_gemm_real_fits(int real_type, int lanes, int N, int K);
 hipError_t igl_launch_gemm_real(const void *rows, int real_type, const float *act, int act_stride,
                                 int lanes, float *out, int out_stride, int N, int K, hipStream_t stream);
 
+/* A 4-bit plane (code bias 8, no zero points) times 9 to 63 lanes on the bf16
+ * matrix cores; no workspace. */
+int igl_gemm_few_fits(int lanes, int N, int K);
+hipError_t igl_launch_gemm_few(const uint8_t *codes, long long row_stride, const float *gains,
+                               int gain_stride, int group_shift, const float *act, int act_stride,
+                               int lanes, float *out, int out_stride, int N, int K,
+                               hipStream_t stream);
+
 int igl_gemv_rows_per_tile(int lanes);
 int igl_gemv_chunk_cols(int lanes, int K, int lds_limit);
 size_t igl_gemv_part_floats(int lanes, int N, int K, int lds_limit);

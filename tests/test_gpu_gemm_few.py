@@ -1,0 +1,49 @@
+"""The few-lane product of 4-bit planes (9 to 63 lanes) against the 64-bit
+product of the same values.
+
+Every product of a term and a code is exact, so an output's error is the
+rounding of its fp32 additions: a product passes at most 12 inside its unit's
+chain, the gain's multiply-add, seven more in a run of eight units, K / 2048
+runs a wave (eight waves share K at least), and 15 across the waves; each at
+most half an ulp of a sum no larger than sum |x w|.
+"""
+import numpy as np
+import pytest
+
+from igllm_amd.backend import make_plane
+
+pytestmark = pytest.mark.gpu
+
+
+# the tiles' edges, K of one unit, not a whole K split, more than one run;
+# wider groups and one gain a row; lanes and outputs with a stride
+@pytest.mark.parametrize("N,K,lanes,group", [
+    (1, 32, 9, 32), (17, 96, 63, 32), (4097, 64, 15, 32), (8193, 128, 16, 64), (1000, 1056, 33, 32),
+    (4100, 544, 31, 544), (6145, 1536, 49, 32), (8192, 2080, 63, 32), (12300, 96, 47, 96), (16400, 64, 63, 32),
+    (300, 6176, 17, 128), (5000, 12288, 12, 32),
+])
+@pytest.mark.parametrize("spread", [False, True])
+def test_few_lanes(backend, N, K, lanes, group, spread):
+    rng = np.random.default_rng(N + K + lanes)
+    stride = (K // 2 + 15) // 16 * 16
+    codes = rng.integers(0, 256, size=(N, stride), dtype=np.uint8)
+    groups = (K + group - 1) // group
+    gains = np.abs(rng.normal(0, 0.02, size=(N, groups))).astype(np.float32)
+    act = rng.normal(size=(lanes, K + 4)).astype(np.float32)
+    if spread:  # the terms' exponent range
+        act *= np.exp2(rng.integers(-60, 60, size=act.shape)).astype(np.float32)
+    cp = backend.attach(make_plane(codes, gains, K, group_size=group))
+    dev_act, dev_out = backend.upload(act), backend.alloc(lanes * (N + 3) * 4)
+    backend.gemv_dev(cp, dev_act, K + 4, lanes, dev_out, N + 3)
+    backend.sync()
+    got = dev_out.get(np.float32, lanes * (N + 3)).reshape(lanes, N + 3)[:, :N]
+    dev_act.free()
+    dev_out.free()
+    backend.detach(cp)
+    value = np.empty((N, K), np.float64)
+    value[:, 0::2] = (codes[:, :K // 2] & 15).astype(np.float64) - 8
+    value[:, 1::2] = (codes[:, :K // 2] >> 4).astype(np.float64) - 8
+    value *= np.repeat(gains.astype(np.float64), group, axis=1)[:, :K]
+    x = act[:, :K].astype(np.float64)
+    bound = (12 + 2 + 7 + K / 2048 + 15) * 2.0 ** -24 * (np.abs(x) @ np.abs(value).T)
+    assert np.all(np.abs(got - x @ value.T) <= bound)
