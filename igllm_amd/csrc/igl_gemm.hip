@@ -376,6 +376,20 @@ __global__ __launch_bounds__(64 * WN * WM * KS) void gemm_codes_kernel(GemmCodes
   for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < NB; ++j) acc[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  // Two terms in the two-a-CU form, which splits K only in two: acc holds the
+  // last kRun steps' groups, sum the runs before, so no output is rounded at
+  // its full size for every group (1536 x 6144 at 1000 lanes 1.1e-7 off the
+  // 64-bit product, the eight-wave form 1.5e-7).  On the one-term forms it cost
+  // 3% and is below bf16's rounding.
+  constexpr bool kRuns = LO && !ROWGAIN && LIM == 80;
+  constexpr int kRun = 8;
+  float4_t sum[kRuns ? MB : 1][kRuns ? NB : 1];
+  if (kRuns) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) sum[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  }
   const uint32_t exp10 = 0x64006400u;  // 1024.0 in both halves
   const half2_t pair_c = as_half2(g.bias_pair);
   // A dword of eight codes k .. k + 7 as the binary16 operand
@@ -408,6 +422,16 @@ __global__ __launch_bounds__(64 * WN * WM * KS) void gemm_codes_kernel(GemmCodes
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (s + AHEAD < steps) issue(s + AHEAD);
+    if (kRuns && s % kRun == 0 && s > 0) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sum[i][j][r] += acc[i][j][r];
+          acc[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
     const uint8_t *st = stage(s);
     half8_t bf[NB][2];
     float gain[NB][2];
@@ -473,6 +497,15 @@ __global__ __launch_bounds__(64 * WN * WM * KS) void gemm_codes_kernel(GemmCodes
       // right behind its own product)
       if (!ROWGAIN) __builtin_amdgcn_sched_barrier(0);
     }
+  }
+
+  if (kRuns) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][j][r] += sum[i][j][r];
   }
 
   // The K split's partial tiles, added in ks order.
@@ -615,12 +648,19 @@ constexpr FormShape kFormsLo[] = {
 };
 
 // A launch takes, of the forms whose K split divides K:
-//   * the 256 x 256 or 128 x 128 form where its tiles fill the 256 CUs;
-//   * else, where the 64 x 64 tiles exceed one round of 256 (one workgroup a
-//     CU at 126 KB of stages), the same tiles in four-wave workgroups, two a
-//     CU at 74-75 KB;
+//   * where the 64 x 64 tiles exceed one round of 256 (one workgroup a CU at
+//     126 KB of stages): of the 256 x 256 (two terms: 256 x 128), the 128 x 128
+//     and the 64 x 64 form in four-wave workgroups, two a CU at 74-75 KB, the
+//     one whose rounds take the least time;
 //   * else, of the 64 x 64, 32 x 64 and 16 x 64 forms, the one with the most
 //     tiles one round holds.
+// A round's time in rounds of the two-a-CU form (512 workgroups; K = 1536, us a
+// round, bf16 / fp32 activations: 15.6 / 20.5; 128 x 128 24.5 / 34.5, form 0 72 /
+// 57): 1.55 / 1.68 and 4.5 / 2.75.  A last round nearly empty costs a whole one,
+// so the widest form that fills the CUs is often not it: 6144 x 1536 at 1000
+// lanes, fp32, 384 tiles of 128 x 128 are two rounds, 79.9 us, 1536 of 64 x 64
+// three, 69.9; 12288 x 1536 at 1000 lanes 120 (form 0) -> 107 (128 x 128); 6144 x
+// 1536 at 2047 lanes 123 -> 110.
 // Against the widest form that filled the CUs (the choice before), replayed,
 // us, bf16 / fp32 activations: 8192 x 2048 at 256 lanes 30.2 / 41.5 -> 27.2 /
 // 35.1 (two a CU); 6144 x 1536 at 128 lanes 22.5 / 30.0 -> 15.0 / 18.7 (64 x 64,
@@ -635,9 +675,21 @@ static int choose_form(int M, int N, int K, int two_terms) {
     const long tn = 16L * forms[f].nb * forms[f].wn, tm = 16L * forms[f].mb * forms[f].wm;
     return ((N + tn - 1) / tn) * ((M + tm - 1) / tm);
   };
-  for (int f = 0; f < 2; ++f)
-    if (divides(f) && tiles(f) >= 256) return f;
-  if (divides(kPairForm) && tiles(kPairForm) > 256) return kPairForm;
+  if (divides(kPairForm) && tiles(kPairForm) > 256) {
+    const double round[] = {two_terms ? 2.75 : 4.5, two_terms ? 1.68 : 1.55};
+    int pick = kPairForm;
+    double least = (double)((tiles(kPairForm) + 511) / 512);
+    for (int f = 1; f >= 0; --f) {
+      const double cost = round[f] * (double)((tiles(f) + 255) / 256);
+      // form 0 sums all of K in one wave: only where its own tiles fill the CUs
+      if (divides(f) && cost < least && (f == 1 || tiles(0) >= 256)) {
+        least = cost;
+        pick = f;
+      }
+    }
+    return pick;
+  }
+  if (divides(0) && tiles(0) >= 256) return 0;
   int best = -1;
   for (int f = 2; f < 5; ++f) {
     if (!divides(f)) continue;
@@ -658,7 +710,8 @@ struct GemmPlan {
 
 // Long rows (K >= 4096) where choose_form ends past the 128 x 128 form take the
 // 64 x 64 form in eight-wave workgroups (at 1024 lanes of 2048 x 8192 the
-// two-a-CU form was no faster: 79.0 against 77.0 us), with K split across
+// two-a-CU form was no faster: 79.0 against 77.0 us; with two terms it is, 1536 x
+// 6144 at 1000 lanes 80.0 against 87.1, and stays), with K split across
 // workgroups into S = 1, 2, 4 or 8 slices: each workgroup then
 // stages K / S of its lanes' activations instead of all of K, for S fp32
 // partial tiles written and folded.  S is the most slices whose workgroups
@@ -678,7 +731,7 @@ struct GemmPlan {
 // (64-256): the partials cost more than the shorter staging saves.
 static GemmPlan choose_plan(int M, int N, int K, int two_terms, bool close) {
   GemmPlan p{choose_form(M, N, K, two_terms), 1};
-  if (close || K < 4096 || p.form < kSplitForm) return p;
+  if (close || K < 4096 || p.form < kSplitForm || (two_terms && p.form == kPairForm)) return p;
   const FormShape &s = (two_terms ? kFormsLo : kForms)[kSplitForm];
   if (K % (kStepK * s.ks)) return p;
   const long tiles = (long)((N + 16 * s.nb * s.wn - 1) / (16 * s.nb * s.wn)) *
