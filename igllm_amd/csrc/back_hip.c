@@ -21,6 +21,10 @@
 #define IGL_GEMV_LANES 8  /* lanes one GEMV launch carries */
 #define IGL_GEMV_Q4_LANES 16 /* lanes one 4-bit GEMV launch carries (the matrix-core form) */
 #define IGL_GEMM_FLOOR 64 /* lanes from which mat_mat takes the MFMA GEMM */
+/* lanes from which a calibrated plane takes the integer GEMM: the level GEMV
+ * forms each lane's sums apart (6144 x 1536, 8 lanes 23 us, 63 lanes 178; the
+ * GEMM 11) */
+#define IGL_LEVEL_FLOOR 5
 
 struct igl_device_plane {
   const void  *codes;
@@ -643,6 +647,17 @@ int igl_plane_lift_dev(igl_desk *desk, const igl_plane *sheet, const float *act_
     desk_fail(st, IGL_FAIL_ARGUMENT);
     return IGL_FAIL_ARGUMENT;
   }
+  /* A calibrated code plane of one gain a row, a few lanes: the integer
+   * matrix cores where the desk's workspace has room or can have (a recording
+   * or a replay keeps it as it is), the same exact sums as the launch below. */
+  if (sheet->enter_gain > 0.0f && sheet->form == IGL_PLANE_CODE && lane_count >= IGL_LEVEL_FLOOR &&
+      lane_count < IGL_GEMM_FLOOR && plane_supported(sheet) == IGL_OKAY && sheet->device && !sheet->device->zeros &&
+      sheet->group_count == 1 && igl_gemm_level_fits(sheet->bit_count, sheet->code_bias, sheet->col_count) &&
+      ((uintptr_t)act_dev & 15u) == 0 && (act_stride & 3) == 0 &&
+      (st->gemm_floats * sizeof(float) >=
+           igl_gemm_level_work_bytes(lane_count, sheet->row_count, sheet->col_count, sheet->bit_count) ||
+       !(st->recording || st->replays_live)))
+    return lift_levels_gemm(st, sheet, act_dev, act_stride, lane_count, out_dev, out_stride);
   /* A calibrated code plane below the GEMM's lane floor: one launch on the
    * activation grid, entry and leave grids fused, the reference's level path
    * (exact integer sums) rather than the float path on quant_step values. */

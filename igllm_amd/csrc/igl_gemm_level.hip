@@ -21,11 +21,12 @@
 // 6 10 14 3 7 11 15; the levels are written in the same order
 // (act_level_kernel), so a lane's sixteen levels and sixteen codes meet.
 //
-// Tile: 256 x 256 a workgroup, eight waves (2 x 4) of 128 x 64 as 8 x 4
-// accumulators; K 128 a step (64 for 8-bit codes, whose stages are twice as
-// large), three LDS stages of levels and codes filled only by global_load_lds
-// two steps ahead.  16-byte chunks of a row are XOR-swizzled (lv_key) so that
-// rows read together by the sixteen lanes of a row tile spread over the banks.
+// Tile: eight waves (2 x 4) of 16 MT lanes x 16 NT rows, 64 x 64 to 256 x 192 a
+// workgroup (level_plan); K 128 a step (64 for 8-bit codes, whose stages are
+// twice as large), three LDS stages of levels and codes filled only by
+// global_load_lds two steps ahead.  16-byte chunks of a row are XOR-swizzled
+// (lv_key) so that rows read together by the sixteen lanes of a row tile spread
+// over the banks.
 // K is cut into slices when the tiles leave CUs idle; slices write int32
 // partials that level_close_kernel adds (exactly, in any order) and closes.
 #include "igl_device.h"
@@ -37,24 +38,27 @@ typedef int32_t int4v_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) void global_void_t;
 
-constexpr int kLvM = 256;
-constexpr int kLvN = 256;
 constexpr int kLvStages = 3;
 constexpr int kLvThreads = 512;
 
-template <int BITS>
+// A workgroup's tile: 2 x 4 waves of 16 MT lanes x 16 NT rows.  Every stage
+// array is padded to whole DMA instructions a wave (a lane past the data loads
+// a valid address into the padding).
+template <int BITS, int MT, int NT>
 struct LevelForm {
+  static constexpr int TM = 32 * MT, TN = 64 * NT;
   static constexpr int K = BITS == 8 ? 64 : 128;        // k a step
   static constexpr int Q = K / 64;                      // products a (row, column) tile a step
   static constexpr int RA = K;                          // bytes of a level row in a stage
   static constexpr int RB = K * BITS / 8;               // bytes of a code row in a stage
-  static constexpr int A_BYTES = kLvM * RA;
-  static constexpr int B_BYTES = kLvN * RB;
+  static constexpr int A_BYTES = (TM * RA + 8191) / 8192 * 8192;
+  static constexpr int B_BYTES = (TN * RB + 8191) / 8192 * 8192;
   static constexpr int STAGE = A_BYTES + B_BYTES;
   static constexpr int LDS = kLvStages * STAGE;
   static constexpr int SHIFT = BITS == 4 ? 4 : BITS == 2 ? 6 : 0;
   static constexpr int A_LOADS = A_BYTES / (8 * 1024);  // 16-byte DMA instructions a wave, levels
   static constexpr int B_LOADS = B_BYTES / (8 * 1024);  // and codes
+  static_assert(LDS <= 160 * 1024, "LDS");
 };
 
 // The swizzle of a row of `RB` bytes: its 16-byte chunk c sits at c ^ key,
@@ -119,19 +123,19 @@ __device__ __forceinline__ int4v_t level_codes(const uint8_t *p, uint32_t code_x
   }
 }
 
-template <int BITS>
-__global__ __launch_bounds__(kLvThreads) void gemm_level_kernel(LevelArgs g) {
-  using F = LevelForm<BITS>;
+template <int BITS, int MT, int NT>
+__global__ __launch_bounds__(kLvThreads, MT * NT > 16 ? 2 : 4) void gemm_level_kernel(LevelArgs g) {
+  using F = LevelForm<BITS, MT, NT>;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_l[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 2;      // 2 wave rows of 128
-  const int wn = wave & 3;       // 4 wave columns of 64
+  const int wm = wave >> 2;      // 2 wave rows of 16 MT
+  const int wn = wave & 3;       // 4 wave columns of 16 NT
   int tile_x, tile_y;
   xcd_tile(tile_x, tile_y);
-  const int m0 = tile_y * kLvM;
-  const int n0 = tile_x * kLvN;
+  const int m0 = tile_y * F::TM;
+  const int n0 = tile_x * F::TN;
   const int steps = g.k_steps;
   const int k_first = blockIdx.z * g.k_steps * F::K;
 
@@ -142,14 +146,14 @@ __global__ __launch_bounds__(kLvThreads) void gemm_level_kernel(LevelArgs g) {
   const int8_t *a_src[F::A_LOADS];
 #pragma unroll
   for (int i = 0; i < F::A_LOADS; ++i) {
-    const int r = (64 / CA) * (F::A_LOADS * wave + i) + lane / CA;
+    const int r = min((64 / CA) * (F::A_LOADS * wave + i) + lane / CA, F::TM - 1);
     const int c = (lane % CA) ^ lv_key<F::RA>(r);
     a_src[i] = g.levels + (size_t)min(m0 + r, g.M - 1) * g.K + k_first + 16 * c;
   }
   const uint8_t *b_src[F::B_LOADS];
 #pragma unroll
   for (int i = 0; i < F::B_LOADS; ++i) {
-    const int r = (64 / CB) * (F::B_LOADS * wave + i) + lane / CB;
+    const int r = min((64 / CB) * (F::B_LOADS * wave + i) + lane / CB, F::TN - 1);
     const int c = (lane % CB) ^ lv_key<F::RB>(r);
     b_src[i] = g.codes + (size_t)min(n0 + r, g.N - 1) * (size_t)g.row_stride + (size_t)k_first * BITS / 8 + 16 * c;
   }
@@ -181,29 +185,29 @@ __global__ __launch_bounds__(kLvThreads) void gemm_level_kernel(LevelArgs g) {
     asm volatile("" ::: "memory");
   };
 
-  int4v_t acc[8][4];
+  int4v_t acc[MT][NT];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = int4v_t{0, 0, 0, 0};
+    for (int j = 0; j < NT; ++j) acc[i][j] = int4v_t{0, 0, 0, 0};
   const int gq = lane >> 4;  // lane group: the step's k-sixteen Q gq .. of product q is 4 q + gq
   const int n = lane & 15;
 
   auto read_rows = [&](const uint8_t *st, int i, int4v_t (&a)[F::Q]) {
 #pragma unroll
     for (int q = 0; q < F::Q; ++q) {
-      const int r = wm * 128 + 16 * i + n;
+      const int r = wm * 16 * MT + 16 * i + n;
       const int c = (4 * q + gq) ^ lv_key<F::RA>(r);
       a[q] = *reinterpret_cast<const int4v_t *>(st + r * F::RA + 16 * c);
     }
   };
-  auto read_codes = [&](const uint8_t *st, int4v_t (&b)[F::Q][4]) {
+  auto read_codes = [&](const uint8_t *st, int4v_t (&b)[F::Q][NT]) {
     const uint8_t *bs = st + F::A_BYTES;
 #pragma unroll
     for (int q = 0; q < F::Q; ++q)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int r = wn * 64 + 16 * j + n;
+      for (int j = 0; j < NT; ++j) {
+        const int r = wn * 16 * NT + 16 * j + n;
         const int s = 4 * q + gq;                      // the k-sixteen's slot of BITS * 2 bytes
         const int byte = s * BITS * 2;                 // logical offset in the row
         const int c = (byte >> 4) ^ lv_key<F::RB>(r);  // its 16-byte chunk, swizzled
@@ -217,20 +221,21 @@ __global__ __launch_bounds__(kLvThreads) void gemm_level_kernel(LevelArgs g) {
     wait_meet(s + 1 < steps);
     if (s + 2 < steps) issue(s + 2);
     const uint8_t *st = stage_of(s);
-    int4v_t bf[F::Q][4];
+    int4v_t bf[F::Q][NT];
     read_codes(st, bf);
     int4v_t a_cur[F::Q], a_next[F::Q];
     read_rows(st, 0, a_cur);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (i + 1 < 8) read_rows(st, i + 1, a_next);
+    for (int i = 0; i < MT; ++i) {
+      if (i + 1 < MT) read_rows(st, i + 1, a_next);
 #pragma unroll
       for (int q = 0; q < F::Q; ++q)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < NT; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bf[q][j], a_cur[q], acc[i][j], 0, 0, 0);
 #pragma unroll
-      for (int q = 0; q < F::Q; ++q) a_cur[q] = a_next[q];
+      for (int q = 0; q < F::Q; ++q)
+        if (i + 1 < MT) a_cur[q] = a_next[q];
     }
   }
 
@@ -238,22 +243,22 @@ __global__ __launch_bounds__(kLvThreads) void gemm_level_kernel(LevelArgs g) {
   // row l % 16 of its row tile and columns 4 (l / 16) .. + 3.
   const bool vec_ok = g.part ? (g.N % 4 == 0) : (g.out_stride % 4 == 0 && ((uintptr_t)g.out & 15u) == 0);
   int32_t *part = g.part ? g.part + (size_t)blockIdx.z * (size_t)g.M * (size_t)g.N : nullptr;
-  // fl(gain * step) of the lane's sixteen columns, loaded before any store
+  // fl(gain * step) of the lane's columns, loaded before any store
   // (the outputs could alias the gains as far as the compiler knows)
-  float gs[4][4];
+  float gs[NT][4];
   const float leave_rcp = g.leave > 0.0f ? level_recip(g.leave) : 0.0f;
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+  for (int j = 0; j < NT; ++j)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) gs[j][r] = g.gains[min(n0 + wn * 64 + j * 16 + 4 * gq + r, g.N - 1)] * g.step;
+    for (int r = 0; r < 4; ++r) gs[j][r] = g.gains[min(n0 + wn * 16 * NT + j * 16 + 4 * gq + r, g.N - 1)] * g.step;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int m = m0 + wm * 128 + i * 16 + n;
+  for (int i = 0; i < MT; ++i) {
+    const int m = m0 + wm * 16 * MT + i * 16 + n;
     if (m >= g.M) continue;
     const bool nan_row = !part && g.nan_rows[m];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int nb = n0 + wn * 64 + j * 16 + 4 * gq;
+    for (int j = 0; j < NT; ++j) {
+      const int nb = n0 + wn * 16 * NT + j * 16 + 4 * gq;
       if (part) {
         if (vec_ok && nb + 3 < g.N) {
           *reinterpret_cast<int4v_t *>(part + (size_t)m * g.N + nb) = acc[i][j];
@@ -349,17 +354,42 @@ __global__ void act_level_kernel(const float *act, int act_stride, int K, float 
 
 static int level_step_k(int bits) { return bits == 8 ? 64 : 128; }
 
-// K slices while the tiles fill under half the CUs: a slice's int32 partials
-// are M x N words each way, and at M = 2048 they cost more than idle CUs do
-// (6144 x 1536, 192 tiles: 47 us unsplit, 86 us in two slices; 2048 x 1536,
-// 64 tiles: 44.6 us in two, 46.2 us unsplit).
-static int level_slices(int M, int N, int K, int bits) {
-  const int tiles = ((M + kLvM - 1) / kLvM) * ((N + kLvN - 1) / kLvN);
+// A launch takes 64 x 64 tiles (lanes x rows) while three workgroups a CU hold
+// them all (768), else 64 x 128 (to 768 tiles, 1536 for 2- and 4-bit codes), else
+// 128 x 128 (to 1024), else 256 x 192.  Many small workgroups a CU hide each
+// other's stages and closes; the widest tile reads the least.  us, the former
+// 256 x 256 tile (K in slices) -> the choice, its neighbours:
+//   6144 x 1536, 4-bit:  64 lanes 16.0 -> 11.0, 500 lanes 38.7 -> 16.7 (64 x 128
+//     17.4), 1000 lanes 47.9 -> 22.6 (64 x 64 26.5, 128 x 128 24.5), 2047 lanes 44.8
+//     -> 38.7 (128 x 128 39.9)
+//   2048 x 1536, 4-bit:  1000 lanes 35.3 -> 14.4 (64 x 128 15.2), 2047 lanes 44.7 ->
+//     21.5 (64 x 64 24.0)
+//   8192 x 2048, 4-bit:  2048 lanes 56.6 -> 52.8 (64 x 128 56.3)
+//   12288 x 6144, 4-bit: 2047 lanes 188 -> 160 (128 x 128 172)
+//   1536 x 6144, 4-bit:  1000 lanes 45.6 -> 31.0; 8-bit 8192 x 2048, 500 lanes 45.6
+//     -> 23.9 (128 x 128 23.9, 64 x 64 31.4)
+// Where those tiles fill under half the CUs K is cut into slices of eight steps
+// and more (their int32 partials and the close cost a launch): 1536 x 6144 at 64
+// lanes 22.1 unsplit, 14.1 in slices; 6144 x 1536 (twelve steps) 11.0 unsplit, 12.2.
+struct LevelShape {
+  int mt, nt, tiles, tiles_8bit;
+};
+constexpr LevelShape kLevelForms[] = {{2, 1, 768, 768}, {2, 2, 1536, 768}, {4, 2, 1024, 1024}, {8, 3, 0, 0}};
+
+struct LevelPlan {
+  int form, slices;
+};
+
+static LevelPlan level_plan(int M, int N, int K, int bits) {
   const int steps = K / level_step_k(bits);
-  int slices = 1;
-  while (slices < 16 && tiles * slices < 128 && steps % (2 * slices) == 0 && steps / (2 * slices) >= 2)
-    slices *= 2;
-  return slices;
+  for (int form = 0;; ++form) {
+    const LevelShape &f = kLevelForms[form];
+    const long tiles = (long)((M + 32 * f.mt - 1) / (32 * f.mt)) * ((N + 64 * f.nt - 1) / (64 * f.nt));
+    if (form < 3 && tiles > (bits == 8 ? f.tiles_8bit : f.tiles)) continue;
+    int slices = 1;
+    while (slices < 16 && tiles * slices < 128 && steps % (2 * slices) == 0 && steps / (2 * slices) >= 8) slices *= 2;
+    return LevelPlan{form, slices};
+  }
 }
 
 static size_t level_levels_bytes(int M, int K) { return ((size_t)M * (size_t)K + 255) & ~(size_t)255; }
@@ -376,24 +406,35 @@ extern "C" int igl_gemm_level_fits(int bits, int code_bias, int K) {
 }
 
 extern "C" size_t igl_gemm_level_work_bytes(int M, int N, int K, int bits) {
-  const int slices = level_slices(M, N, K, bits);
+  const int slices = level_plan(M, N, K, bits).slices;
   return level_levels_bytes(M, K) + level_flag_bytes(M) +
          (slices > 1 ? (size_t)slices * (size_t)M * (size_t)N * sizeof(int32_t) : 0);
 }
 
-template <int BITS>
-static hipError_t gemm_level_launch(const LevelArgs &a, int slices, hipStream_t stream) {
-  const size_t lds = (size_t)LevelForm<BITS>::LDS;
-  static bool granted = false;
+template <int BITS, int F>
+static hipError_t gemm_level_form(const LevelArgs &a, int slices, hipStream_t stream) {
+  constexpr int MT = kLevelForms[F].mt, NT = kLevelForms[F].nt;
+  using L = LevelForm<BITS, MT, NT>;
+  static bool granted = false;  // the dynamic LDS a kernel asks for is granted once
   if (!granted) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_level_kernel<BITS>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_level_kernel<BITS, MT, NT>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, L::LDS);
     if (e != hipSuccess) return e;
     granted = true;
   }
-  dim3 grid((a.N + kLvN - 1) / kLvN, (a.M + kLvM - 1) / kLvM, slices);
-  hipLaunchKernelGGL((gemm_level_kernel<BITS>), grid, dim3(kLvThreads), lds, stream, a);
+  dim3 grid((a.N + L::TN - 1) / L::TN, (a.M + L::TM - 1) / L::TM, slices);
+  hipLaunchKernelGGL((gemm_level_kernel<BITS, MT, NT>), grid, dim3(kLvThreads), (size_t)L::LDS, stream, a);
   return hipGetLastError();
+}
+
+template <int BITS>
+static hipError_t gemm_level_launch(const LevelArgs &a, const LevelPlan &p, hipStream_t stream) {
+  switch (p.form) {
+    case 0: return gemm_level_form<BITS, 0>(a, p.slices, stream);
+    case 1: return gemm_level_form<BITS, 1>(a, p.slices, stream);
+    case 2: return gemm_level_form<BITS, 2>(a, p.slices, stream);
+    default: return gemm_level_form<BITS, 3>(a, p.slices, stream);
+  }
 }
 
 extern "C" hipError_t igl_launch_gemm_level(const float *act, int act_stride, const uint8_t *codes,
@@ -405,7 +446,8 @@ extern "C" hipError_t igl_launch_gemm_level(const float *act, int act_stride, co
       ((uintptr_t)codes & 15u) || ((uintptr_t)act & 15u) || act_stride % 4 || (M > 1 && act_stride < K) ||
       (M > 1 && out_stride < N))
     return hipErrorInvalidValue;
-  const int slices = level_slices(M, N, K, bits);
+  const LevelPlan plan = level_plan(M, N, K, bits);
+  const int slices = plan.slices;
   int8_t *levels = reinterpret_cast<int8_t *>(work);
   int32_t *nan_rows = reinterpret_cast<int32_t *>(reinterpret_cast<uint8_t *>(work) + level_levels_bytes(M, K));
   int32_t *part = slices > 1 ? reinterpret_cast<int32_t *>(reinterpret_cast<uint8_t *>(nan_rows) +
@@ -441,9 +483,9 @@ extern "C" hipError_t igl_launch_gemm_level(const float *act, int act_stride, co
   a.N = N;
   a.K = K;
   a.k_steps = K / level_step_k(bits) / slices;
-  e = bits == 4 ? gemm_level_launch<4>(a, slices, stream)
-      : bits == 2 ? gemm_level_launch<2>(a, slices, stream)
-                  : gemm_level_launch<8>(a, slices, stream);
+  e = bits == 4 ? gemm_level_launch<4>(a, plan, stream)
+      : bits == 2 ? gemm_level_launch<2>(a, plan, stream)
+                  : gemm_level_launch<8>(a, plan, stream);
   if (e != hipSuccess || slices == 1) return e;
   const int shift = bits == 4 ? 4 : bits == 2 ? 6 : 0;
   hipLaunchKernelGGL(level_close_kernel, dim3((N + 255) / 256, M), dim3(256), 0, stream, part, slices, M, N, shift,

@@ -1,0 +1,45 @@
+"""The integer GEMM of calibrated planes (five lanes and more) against each
+lane's own launch.
+
+One lane takes the level GEMV, whose sums are the reference's to the bit
+(test_plane_lift_level_bitexact); every sum of the GEMM is an exact integer and
+its row close the same, so the outputs are equal, bit for bit, whatever the
+tile or the K slices.
+"""
+import numpy as np
+import pytest
+
+from igllm_amd.backend import make_plane
+
+pytestmark = pytest.mark.gpu
+
+
+# each tile's edges (64 x 64, 64 x 128, 128 x 128, 256 x 192: lanes x rows), K
+# slices, one step, lanes below and past the GEMM's former floor
+@pytest.mark.parametrize("bits", [2, 4, 8])
+@pytest.mark.parametrize("N,K,lanes", [(16, 128, 5), (300, 2048, 63), (96, 6144, 64), (1000, 256, 65), (4112, 384, 767),
+                                       (6160, 128, 1030), (12304, 128, 1990)])
+def test_lanes_equal_single_lanes(backend, bits, N, K, lanes):
+    rng = np.random.default_rng(N + K + lanes + bits)
+    codes = rng.integers(0, 256, size=(N, (K * bits // 8 + 15) // 16 * 16), dtype=np.uint8)
+    gains = (rng.random((N, 1)) * 0.02 + 0.01).astype(np.float32)
+    cp = make_plane(codes, gains, K, group_size=K, bits=bits)
+    cp.plane.enter_gain, cp.plane.leave_gain = 0.04, 0.1 * 4 ** (bits // 4)
+    backend.attach(cp)
+    act = rng.normal(size=(lanes, K + 4)).astype(np.float32)
+    dev_act, out, one = backend.upload(act), backend.alloc(lanes * (N + 4) * 4), backend.alloc(N * 4)
+
+    class Lane:
+        ptr = 0
+
+    backend.plane_lift_dev(cp, dev_act, K + 4, lanes, out, N + 4)
+    backend.sync()
+    got = out.get(np.float32, lanes * (N + 4)).reshape(lanes, N + 4)[:, :N]
+    for lane in sorted({0, 1, 15, 16, 63, 64, lanes // 2, lanes - 1} & set(range(lanes))):
+        Lane.ptr = dev_act.ptr + 4 * (K + 4) * lane
+        backend.plane_lift_dev(cp, Lane, K, 1, one, N)
+        backend.sync()
+        assert np.array_equal(got[lane].view(np.uint32), one.get(np.float32, N).view(np.uint32)), lane
+    for b in (dev_act, out, one):
+        b.free()
+    backend.detach(cp)
