@@ -119,8 +119,8 @@ struct igl_engine {
   int graph_on, graph_ready, graph_tried;
   hipGraphExec_t graph;
   /* a speculative block of `count` lanes as one captured graph per count
-   * (blocks below the GEMM's lane floor, whose launches use only buffers
-   * fixed at open and attach): ctl_host[0 .. count] is copied to ctl_dev */
+   * (blocks below the GEMM's lane floor; captured anew once the desk's
+   * workspace moves): ctl_host[0 .. count] is copied to ctl_dev */
   int32_t *ctl_host;  /* pinned: the block's position and ids */
   unsigned graph_gen; /* the desk's workspace generation the graphs were captured at */
   hipGraphExec_t guess_graph[ENG_GUESS_LIMIT + 1];
@@ -1334,9 +1334,11 @@ static int capture_guess(igl_engine *e, int count) {
  *
  * With graphs on, a block of fewer lanes than the GEMM's floor replays one
  * graph captured for its lane count (the first block of each count runs as
- * enqueued, with the same grid, then is captured): every projection of such a
- * block is a GEMV, whose launches use only the workspace reserved at attach,
- * so no captured address can move.  Larger blocks run as enqueued. */
+ * enqueued, with the same grid, then is captured): the launches of such
+ * a block use the workspace reserved at attach and, for calibrated planes from
+ * five lanes, the GEMM workspace the enqueued block has grown; should the desk
+ * grow it again, its generation moves and the graphs are captured anew.
+ * Larger blocks run as enqueued. */
 int igl_engine_guess(igl_engine *e, const int32_t *ids, int count, int32_t *picks_out,
                      float *margins_out) {
   if (!e || !ids || count < 1 || count > e->guess_limit) return IGL_FAIL_ARGUMENT;

@@ -319,8 +319,9 @@ void igl_zero_unpack(const uint32_t *words, int groups, int rows, int bits, int8
  * activations and the byte key/value cache in HBM: ids in, greedy picks out.
  * Loads config.json + model.safetensors from `folder` (4-bit planes, one KV
  * head per 8 query heads, byte cache scales).  `lane_limit` lanes run per pass
- * (the reference's is 16); `precise` keeps every projection on the fp32
- * activation GEMV, otherwise batches of 64+ lanes take the MFMA GEMM. */
+ * (the reference's is 16); `precise` keeps every pass below 64
+ * lanes (the GEMV and the few-lane products), otherwise batches of 64+ lanes
+ * take the MFMA GEMM. */
 typedef struct igl_engine igl_engine;
 int  igl_engine_open(igl_engine **engine_out, igl_desk *desk, const char *folder,
                      int window_limit, int lane_limit, int precise);
