@@ -669,17 +669,26 @@ __global__ __launch_bounds__(256) void attend_split_kernel(AttendArgs a) {
 // What bounds it: a chunk's chain between the two barriers (decode, products,
 // the exchanged sums, the exponentials; 6200 cycles a chunk of 512-dim heads at
 // 32 rows, 2000 of them products on each SIMD).  At 2047 lanes, us, against one
-// workgroup a lane: 2048 positions of 512-dim heads 450 -> 118 (69 GFLOP of
-// products, two terms each: 580 TFLOP/s), a 512 window of 256-dim heads 104 -> 37;
-// 511 lanes 57 -> 22.  Four waves of 128 dims, two workgroups a CU: 129 us (a
-// chunk's chain is 8800 cycles, and the longest tile's chunks bound the launch);
-// the keys in registers instead of LDS spilled (166 us).
+// workgroup a lane: 2048 positions of 512-dim heads 450 -> 101 (69 GFLOP of
+// products, two terms each: 680 TFLOP/s), a 512 window of 256-dim heads 104 -> 34;
+// 511 lanes 57 -> 22.  Against an earlier form at 118 us: four waves of 128 dims,
+// two workgroups a CU, 129 (a chunk's chain is 8800 cycles, and the longest
+// tile's chunks bound the launch); the keys in registers instead of LDS spilled
+// (166).
 //
 // Per chunk: scores S = q_lo . K^T + q_hi . K^T (the waves' sums added in wave
-// order), the rows' peak and total updated online, probabilities to LDS as two
-// binary16 terms, and blend = blend e^(old peak - peak) + (p_lo + p_hi) . V,
-// each chunk's products formed from zero.  Positions a lane does not see have
-// probability zero in its rows.
+// order), probabilities p = e^(S - base) to LDS as two binary16 terms, and total
+// and blend = blend e^(old base - base) + (p_lo + p_hi) . V, each chunk's products
+// formed from zero.  A row's base stays while it is at or below the chunk's
+// peak, by ten at most (p below 2^15), else it is the chunk's peak, so p's two
+// terms lose no more than against that peak: half of 2^-24 of the chunk's
+// largest.  Against the running peak, the weights far below an early position's
+// fall under binary16's range: one position 18 above 1000-1900 others, its own
+// value zero, left the blend 12% (256 dims) and 40% (512) off, 4.5% and 8.5%
+// from the chunk that holds it alone, as here.  No base is more than forty under
+// the largest peak, so the scaled sums stay in fp32's range.  It costs 1% of a
+// launch (99.3 -> 100.7 us at 2047 lanes of 512 dims).  Positions a lane does not
+// see have probability zero in its rows.
 typedef __attribute__((address_space(3))) void attend_lds_t;
 typedef __attribute__((address_space(1))) const void attend_global_t;
 
@@ -761,12 +770,12 @@ __global__ __launch_bounds__(HEAD, 2) void attend_tile_kernel(AttendArgs a) {
   const bool split = gridDim.z > 1;
 
   // the softmax's row of this thread, its lane's visible positions (relative
-  // to start) and its running peak and total
+  // to start), its largest peak, its base and its running total
   const int row = min(tid / TPR, ROWS - 1);
   const int li = min(row / kAttendGroup, ln - 1);
   const int see_end = pos0 + li - start;  // inclusive
   const int see_first = a.window > 0 ? max(0, pos0 + li + 1 - a.window) - start : 0;
-  float run_m = -INFINITY, run_l = 0.0f;
+  float top = -INFINITY, run_m = -INFINITY, run_l = 0.0f;
 
   const int ring0 = start % a.cache_span;
   // t < span < 2 cache_span (the host takes this form past 64 visible positions)
@@ -938,7 +947,9 @@ __global__ __launch_bounds__(HEAD, 2) void attend_tile_kernel(AttendArgs a) {
       peak = fmaxf(peak, dpp_move<0x4E>(peak));
       if (TPR >= 8) peak = fmaxf(peak, dpp_move<0x141>(peak));
       if (TPR >= 16) peak = fmaxf(peak, dpp_move<0x140>(peak));
-      const float m = fmaxf(run_m, peak);
+      top = fmaxf(top, peak);
+      const float over = peak - run_m;
+      const float m = over >= 0.0f && over <= 10.0f ? run_m : fmaxf(peak, top - 40.0f);
       const float keep = run_m != -INFINITY ? __expf(run_m - m) : 0.0f;
       float total = 0.0f;
       _Float16 hi[PPT], lo[PPT];
