@@ -1131,7 +1131,7 @@ __global__ __launch_bounds__(256) void attend_fold_kernel(const float *part_out_
       T += red_l[i];
     }
     blend_all[(size_t)lane_id * o_stride + (size_t)h * head_size + blockIdx.z * DIMS + d] =
-        T > 0.0f ? A * (1.0f / T) : 0.0f;
+        T == 0.0f ? 0.0f : A * (1.0f / T);  // NaN: a lane whose scores are
   }
 }
 

@@ -1,4 +1,5 @@
-"""Attention whose scores are not flat: a sink position far above the others.
+"""Attention whose scores are not flat: a sink position far above the others,
+and a lane whose query holds a NaN.
 
 A trained model puts most of a head's weight on one early position.  The
 others' weights are then e^-10 to e^-18 of it, and where the sink's own value
@@ -82,3 +83,29 @@ def test_sink(backend, lanes, place, head, fmt, peak, value):
         err = np.abs(got[lane] - w @ v / total)
         bound = U * (each @ np.abs(v)) / total
         assert np.all(err <= bound), (lane, float((err / bound).max()))
+
+
+# tiles, and tiles folded from segments
+@pytest.mark.parametrize("lanes,place,head", [(16, 300, 512), (100, 1900, 256), (130, 0, 512), (600, 0, 512),
+                                              (1030, 0, 512)])
+def test_nan_query(backend, lanes, place, head):
+    """A NaN in one head of one lane's query: that head's blend is NaN,
+    whatever form the launch takes, and no other output changes."""
+    print("case nan query", lanes, place, head, flush=True)
+    rng = np.random.default_rng(lanes)
+    ring, scale = place + lanes, 4.0 / 127.0
+    rings = [backend.upload(rng.integers(0, 256, size=(ring, head), dtype=np.uint8)) for _ in range(2)]
+    query = rng.normal(size=(lanes, 8, head)).astype(np.float32)
+    lane = lanes // 2
+    bad = query.copy()
+    bad[lane, 3, 7] = np.nan
+    q_dev, bad_dev, out = backend.upload(query), backend.upload(bad), backend.alloc(query.nbytes)
+    try:
+        want = attend(backend, rings, 1, scale, ring, head, q_dev, lanes, place, 0, out)
+        got = attend(backend, rings, 1, scale, ring, head, bad_dev, lanes, place, 0, out)
+    finally:
+        for b in rings + [q_dev, bad_dev, out]:
+            b.free()
+    assert np.isnan(got[lane, 3]).all(), got[lane, 3, :4]
+    got[lane, 3] = want[lane, 3]
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
