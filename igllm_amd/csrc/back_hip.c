@@ -64,6 +64,9 @@ struct igl_desk_state {
   size_t part_floats;
   float *work_dev;
   size_t work_floats;
+  /* partials of the attention's wide launches (igl_attend_wide):
+   * IGL_ATTEND_FIXED_FLOATS floats, held from open to close */
+  float *attend_dev;
   float *quant_dev;   /* plane_lift: the activations on the plane's entry grid */
   size_t quant_floats;
   /* plane_lift's prefill on the grid: widened codes, unit gains, level sums,
@@ -726,6 +729,7 @@ int igl_attend_lanes_dev(igl_desk *desk, const uint8_t *key_store, const uint8_t
                          int lane_stride, int place_first, int window, int lane_count,
                          float score_scale, float *blend_out_dev) {
   igl_desk_state *st = desk ? desk->state : NULL;
+  float *work;
   size_t need;
   int code;
   if (!st) return IGL_FAIL_STATE;
@@ -733,17 +737,22 @@ int igl_attend_lanes_dev(igl_desk *desk, const uint8_t *key_store, const uint8_t
                            head_size, query_dev, lane_stride, place_first, window, lane_count,
                            blend_out_dev)) != IGL_OKAY)
     return code;
-  need = igl_attend_work_floats(place_first, window, lane_count, kv_count * group_share, head_size);
-  if (grow_dev(st, &st->work_dev, &st->work_floats, need) != IGL_OKAY) return IGL_FAIL_MEMORY;
+  work = st->attend_dev;
+  if (!igl_attend_wide(place_first, window, lane_count)) {
+    need = igl_attend_work_floats(place_first, window, lane_count, kv_count * group_share, head_size);
+    if (grow_dev(st, &st->work_dev, &st->work_floats, need) != IGL_OKAY) return IGL_FAIL_MEMORY;
+    work = st->work_dev;
+  }
   return hip_check(st, igl_launch_attend(key_store, value_store, format, key_scale, value_scale,
                                          cache_span, kv_count * head_size, kv_count, group_share,
                                          head_size, query_dev, lane_stride, place_first, NULL,
-                                         window, lane_count, score_scale, blend_out_dev,
-                                         st->work_dev, st->stream));
+                                         window, lane_count, score_scale, blend_out_dev, work,
+                                         st->stream));
 }
 
 /* The same kernels with the partials in the fixed per-device array
- * (igl_attend.hip); nothing is allocated or freed. */
+ * (igl_attend.hip), a wide launch's in the desk's own; nothing is allocated or
+ * freed. */
 int igl_attend_lanes_fixed_dev(igl_desk *desk, const uint8_t *key_store,
                                const uint8_t *value_store, int format, float key_scale,
                                float value_scale, int cache_span, int kv_count, int group_share,
@@ -758,14 +767,17 @@ int igl_attend_lanes_fixed_dev(igl_desk *desk, const uint8_t *key_store,
                            head_size, query_dev, lane_stride, place_first, window, lane_count,
                            blend_out_dev)) != IGL_OKAY)
     return code;
-  if (igl_attend_work_floats(place_first, window, lane_count, kv_count * group_share, head_size) >
-      (size_t)IGL_ATTEND_FIXED_FLOATS) {
-    desk_fail(st, IGL_FAIL_SUPPORT);
-    return IGL_FAIL_SUPPORT;
-  }
-  if (!(work = igl_attend_fixed_ptr(st->device))) {
-    desk_fail(st, IGL_FAIL_STATE);
-    return IGL_FAIL_STATE;
+  work = st->attend_dev;
+  if (!igl_attend_wide(place_first, window, lane_count)) {
+    if (igl_attend_work_floats(place_first, window, lane_count, kv_count * group_share, head_size) >
+        (size_t)IGL_ATTEND_FIXED_FLOATS) {
+      desk_fail(st, IGL_FAIL_SUPPORT);
+      return IGL_FAIL_SUPPORT;
+    }
+    if (!(work = igl_attend_fixed_ptr(st->device))) {
+      desk_fail(st, IGL_FAIL_STATE);
+      return IGL_FAIL_STATE;
+    }
   }
   return hip_check(st, igl_launch_attend(key_store, value_store, format, key_scale, value_scale,
                                          cache_span, kv_count * head_size, kv_count, group_share,
@@ -1038,7 +1050,8 @@ int igl_back_open(igl_desk *desk, int device_index, int sum_limit, int col_limit
       hipEventCreate(&st->mark[0]) != hipSuccess || hipEventCreate(&st->mark[1]) != hipSuccess ||
       hipMalloc((void **)&st->act_dev, (size_t)st->lane_limit * st->col_limit * sizeof(float)) != hipSuccess ||
       hipHostMalloc((void **)&st->act_pin, (size_t)st->lane_limit * st->col_limit * sizeof(float),
-                    hipHostMallocDefault) != hipSuccess) {
+                    hipHostMallocDefault) != hipSuccess ||
+      hipMalloc((void **)&st->attend_dev, IGL_ATTEND_FIXED_FLOATS * sizeof(float)) != hipSuccess) {
     desk->state = st;
     igl_back_close(desk);
     return IGL_FAIL_DEVICE;
@@ -1065,6 +1078,7 @@ void igl_back_close(igl_desk *desk) {
   if (st->out_pin) (void)hipHostFree(st->out_pin);
   if (st->part_dev) (void)hipFree(st->part_dev);
   if (st->work_dev) (void)hipFree(st->work_dev);
+  if (st->attend_dev) (void)hipFree(st->attend_dev);
   if (st->quant_dev) (void)hipFree(st->quant_dev);
   if (st->wide_dev) (void)hipFree(st->wide_dev);
   if (st->ones_dev) (void)hipFree(st->ones_dev);

@@ -1464,13 +1464,17 @@ extern "C" size_t igl_attend_prep_work_floats(int place_bound, int window, int h
   return (size_t)lanes * blocks * (size_t)kAttendGroup * ((size_t)head_size + 2);
 }
 
+extern "C" int igl_attend_wide(int place0, int window, int lanes) {
+  return lanes >= kAttendWideLanes && attend_blocks(place0, window, lanes) > 1;
+}
+
 // Floats of workspace igl_launch_attend needs for the same arguments.
 extern "C" size_t igl_attend_work_floats(int place0, int window, int lanes, int head_count,
                                          int head_size) {
   const size_t blocks = (size_t)attend_blocks(place0, window, lanes);
-  // from kAttendWideLanes lanes, more than one chunk: the tiles' segments, or
-  // no partials (below, the tiles' segments take no more than the chunks)
-  if (lanes >= kAttendWideLanes && blocks > 1) {
+  // the tiles' segments, or no partials (below kAttendWideLanes the tiles'
+  // segments take no more than the chunks)
+  if (igl_attend_wide(place0, window, lanes)) {
     const int segments = attend_tile_plan(place0, window, lanes, head_count, head_size).segments;
     return segments == 1 ? 0 : (size_t)lanes * segments * (size_t)head_count * ((size_t)head_size + 2);
   }

@@ -180,6 +180,9 @@ hipError_t igl_launch_gemm_q4(const void *act, int act_bf16, int act_stride, con
                               void *work, const igl_gemm_close *close, hipStream_t stream);
 
 size_t igl_attend_work_floats(int place0, int window, int lanes, int head_count, int head_size);
+/* Whether a launch is one of the wide ones (64 lanes and more, spans past 64
+ * positions), whose partials IGL_ATTEND_FIXED_FLOATS floats always hold. */
+int igl_attend_wide(int place0, int window, int lanes);
 /* The device address of the fixed attention workspace on `device`
  * (IGL_ATTEND_FIXED_FLOATS floats), resolved once per device with it current
  * (igl_back_open); NULL before. */

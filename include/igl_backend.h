@@ -206,12 +206,16 @@ int igl_attend_lanes_dev(igl_desk *desk, const uint8_t *key_store, const uint8_t
  * whose chunk partials live in a fixed array of IGL_ATTEND_FIXED_FLOATS floats
  * (8 MiB) that each GPU holds from the library's load until the process ends,
  * instead of in the desk's grow-only workspace.  It allocates and frees
- * nothing.  A call whose partials exceed the array (at most
+ * nothing.  Calls of 64 lanes and more whose spans pass 64 positions keep what
+ * partials they have in 8 MiB of the desk's own, in either entry: they grow
+ * nothing and always fit.  Of the others, a call whose partials exceed the
+ * array (at most
  * lane_count * kv_count * group_share * (head_size + 2) * ceil(span / 32)
  * floats, span the longest lane's) is refused with IGL_FAIL_SUPPORT before
  * anything is launched.  Every call on one GPU shares that GPU's array and
  * nothing in it needs to start at zero (each partial is written before it is
- * read); calls that overlap on one GPU (two desks, or two streams) race. */
+ * read); calls that use it and overlap on one GPU (two desks, or two streams)
+ * race. */
 #define IGL_ATTEND_FIXED_FLOATS (1u << 21)
 int igl_attend_lanes_fixed_dev(igl_desk *desk, const uint8_t *key_store,
                                const uint8_t *value_store, int format, float key_scale,

@@ -45,6 +45,18 @@ def test_every_launch_fits_the_engine_allocation(lib, window_limit, lane_limit):
     assert worst <= have, (worst, have)
 
 
+@pytest.mark.parametrize("kv", [1, 2, 4])
+@pytest.mark.parametrize("head", [256, 512])
+def test_wide_launches_fit_the_fixed_array(lib, head, kv):
+    """Every launch of 64 lanes and more over more than one chunk keeps its
+    partials in IGL_ATTEND_FIXED_FLOATS floats."""
+    for window in (0, 65, 512, 8192):
+        for lanes in (64, 65, 100, 127, 200, 512, 1030, 2048, 5000):
+            for place in list(range(0, 400, 7)) + list(range(400, 40000, 501)):
+                need = lib.igl_attend_work_floats(place, window, lanes, kv * HEADS, head)
+                assert not lib.igl_attend_wide(place, window, lanes) or need <= 1 << 21, (window, lanes, place)
+
+
 def test_longest_span_alone_falls_short(lib):
     """Sizing by a decode step at the last position, or by a full batch ending
     there, is smaller than a 16-lane batch ending at position 8191 of a
