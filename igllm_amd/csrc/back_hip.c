@@ -145,24 +145,24 @@ int igl_desk_error_take(igl_desk *desk) {
   return code;
 }
 
-/* Grows a device buffer to at least `floats`; used only at load time or on
- * the first call that needs more room. */
-static int grow_dev(igl_desk_state *st, float **buf, size_t *have, size_t floats) {
+/* Grows a device buffer to at least `floats`, or says why not; used only at
+ * load time or on the first call that needs more room. */
+static int try_grow_dev(igl_desk_state *st, float **buf, size_t *have, size_t floats) {
   void *fresh = NULL;
   if (*have >= floats) return IGL_OKAY;
-  if (st->recording || st->replays_live) {
-    desk_fail(st, IGL_FAIL_STATE);
-    return IGL_FAIL_STATE;
-  }
-  if (hipMalloc(&fresh, floats * sizeof(float)) != hipSuccess) {
-    desk_fail(st, IGL_FAIL_MEMORY);
-    return IGL_FAIL_MEMORY;
-  }
+  if (st->recording || st->replays_live) return IGL_FAIL_STATE;
+  if (hipMalloc(&fresh, floats * sizeof(float)) != hipSuccess) return IGL_FAIL_MEMORY;
   if (*buf) (void)hipFree(*buf);
   *buf = (float *)fresh;
   *have = floats;
   st->generation += 1;
   return IGL_OKAY;
+}
+
+static int grow_dev(igl_desk_state *st, float **buf, size_t *have, size_t floats) {
+  const int code = try_grow_dev(st, buf, have, floats);
+  if (code != IGL_OKAY) desk_fail(st, code);
+  return code;
 }
 
 static int grow_out(igl_desk_state *st, size_t floats) {
@@ -251,10 +251,24 @@ static size_t plane_part_floats(const igl_desk_state *st, const igl_plane *sheet
   return most;
 }
 
+/* Calibrated code planes of one gain a row and no zero points whose width the
+ * integer GEMM takes, and the workspace it needs for `lanes`. */
+static int plane_is_level(const igl_plane *sheet) {
+  return sheet->enter_gain > 0.0f && sheet->form == IGL_PLANE_CODE && sheet->group_count == 1 && !sheet->bias_data &&
+         igl_gemm_level_fits(sheet->bit_count, sheet->code_bias, sheet->col_count);
+}
+
+static size_t level_floats(const igl_plane *sheet, int lanes) {
+  return (igl_gemm_level_work_bytes(lanes, sheet->row_count, sheet->col_count, sheet->bit_count) + 3) / 4;
+}
+
 static int plane_reserve(igl_desk_state *st, const igl_plane *sheet) {
   size_t part = plane_part_floats(st, sheet);
   size_t out = (size_t)st->lane_limit * (size_t)sheet->row_count;
   if (part && grow_dev(st, &st->part_dev, &st->part_floats, part) != IGL_OKAY) return IGL_FAIL_MEMORY;
+  /* where there is no room for it, few-lane lifts take the level GEMV */
+  if (plane_is_level(sheet))
+    (void)try_grow_dev(st, &st->gemm_dev, &st->gemm_floats, level_floats(sheet, IGL_GEMM_FLOOR - 1));
   return grow_out(st, out);
 }
 
@@ -651,15 +665,13 @@ int igl_plane_lift_dev(igl_desk *desk, const igl_plane *sheet, const float *act_
     return IGL_FAIL_ARGUMENT;
   }
   /* A calibrated code plane of one gain a row, a few lanes: the integer
-   * matrix cores where the desk's workspace has room or can have (a recording
-   * or a replay keeps it as it is), the same exact sums as the launch below. */
-  if (sheet->enter_gain > 0.0f && sheet->form == IGL_PLANE_CODE && lane_count >= IGL_LEVEL_FLOOR &&
-      lane_count < IGL_GEMM_FLOOR && plane_supported(sheet) == IGL_OKAY && sheet->device && !sheet->device->zeros &&
-      sheet->group_count == 1 && igl_gemm_level_fits(sheet->bit_count, sheet->code_bias, sheet->col_count) &&
+   * matrix cores, the same exact sums as the launch below.  The workspace for it
+   * was reserved with the plane: nothing grows here, so a call can be captured
+   * and moves no generation. */
+  if (lane_count >= IGL_LEVEL_FLOOR && lane_count < IGL_GEMM_FLOOR && plane_is_level(sheet) &&
+      plane_supported(sheet) == IGL_OKAY && sheet->device && !sheet->device->zeros &&
       ((uintptr_t)act_dev & 15u) == 0 && (act_stride & 3) == 0 &&
-      (st->gemm_floats * sizeof(float) >=
-           igl_gemm_level_work_bytes(lane_count, sheet->row_count, sheet->col_count, sheet->bit_count) ||
-       !(st->recording || st->replays_live)))
+      st->gemm_floats >= level_floats(sheet, lane_count))
     return lift_levels_gemm(st, sheet, act_dev, act_stride, lane_count, out_dev, out_stride);
   /* A calibrated code plane below the GEMM's lane floor: one launch on the
    * activation grid, entry and leave grids fused, the reference's level path

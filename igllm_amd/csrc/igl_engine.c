@@ -1334,10 +1334,9 @@ static int capture_guess(igl_engine *e, int count) {
  *
  * With graphs on, a block of fewer lanes than the GEMM's floor replays one
  * graph captured for its lane count (the first block of each count runs as
- * enqueued, with the same grid, then is captured): the launches of such
- * a block use the workspace reserved at attach and, for calibrated planes from
- * five lanes, the GEMM workspace the enqueued block has grown; should the desk
- * grow it again, its generation moves and the graphs are captured anew.
+ * enqueued, with the same grid, then is captured): the launches of such a
+ * block use only the workspace reserved at attach; should the desk grow it for
+ * a larger pass, its generation moves and the graphs are captured anew.
  * Larger blocks run as enqueued. */
 int igl_engine_guess(igl_engine *e, const int32_t *ids, int count, int32_t *picks_out,
                      float *margins_out) {

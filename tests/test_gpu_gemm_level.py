@@ -6,10 +6,12 @@ One lane takes the level GEMV, whose sums are the reference's to the bit
 its row close the same, so the outputs are equal, bit for bit, whatever the
 tile or the K slices.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
-from igllm_amd.backend import make_plane
+from igllm_amd.backend import Backend, make_plane
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +45,42 @@ def test_lanes_equal_single_lanes(backend, bits, N, K, lanes):
     for b in (dev_act, out, one):
         b.free()
     backend.detach(cp)
+
+
+def test_few_lanes_grow_nothing():
+    """The workspace of 5 to 63 lanes is reserved with the plane: a first lift,
+    whatever its lanes, reallocates nothing (the desk's generation stays), and
+    a live replay changes no bit of it."""
+    b = Backend(device=0, sum_limit=1024, col_limit=16384, lane_limit=16)
+    try:
+        N, K = 96, 6144  # K in slices: the most workspace
+        rng = np.random.default_rng(3)
+        codes = rng.integers(0, 256, size=(N, K // 2), dtype=np.uint8)
+        cp = make_plane(codes, np.full((N, 1), 0.02, np.float32), K, group_size=K)
+        cp.plane.enter_gain, cp.plane.leave_gain = 0.04, 0.1
+        b.attach(cp)
+        act, out = b.upload(rng.normal(size=(63, K)).astype(np.float32)), b.alloc(63 * N * 4)
+        before = b.lib.igl_desk_generation(ctypes.byref(b.desk))
+        got = []
+        for lanes in (5, 37, 63):
+            b.plane_lift_dev(cp, act, K, lanes, out, N)
+            b.sync()
+            got.append(out.get(np.float32, lanes * N))
+        b.record_begin()
+        b.plane_lift_dev(cp, act, K, 37, out, N)
+        replay = b.record_end()
+        for lanes, want in zip((5, 37, 63), got):
+            out.put(np.zeros(63 * N, np.float32))
+            b.plane_lift_dev(cp, act, K, lanes, out, N)
+            b.sync()
+            assert np.array_equal(out.get(np.float32, lanes * N).view(np.uint32), want.view(np.uint32))
+        b.replay_run(replay)
+        b.sync()
+        assert np.array_equal(out.get(np.float32, 37 * N).view(np.uint32), got[1].view(np.uint32))
+        b.replay_free(replay)
+        assert b.lib.igl_desk_generation(ctypes.byref(b.desk)) == before
+        b.detach(cp)
+        act.free()
+        out.free()
+    finally:
+        b.close()
