@@ -11,7 +11,8 @@
 // An fp32 activation is three bf16 terms exactly (split3) and a code less its
 // bias one, so every product is exact and nothing of the activations passes
 // through memory first: no workspace, one launch.  A unit's three products
-// are chained from zero, the smallest term first.
+// are chained from zero, the smallest term first.  Activations whose terms or
+// unit sums leave that range are formed again (few_dot).
 //
 // Tiling as gemm_real_kernel's: WN x WM x KS waves own TN x TM of C, K in LDS
 // stages of KS units filled by the LDS DMA, wave group ks takes a stage's
@@ -64,6 +65,36 @@ __device__ __forceinline__ bf8_t code_terms(uint32_t d) {
   for (int i = 0; i < 4; ++i)
     p[i] = high_pair((float)(v << (28 - 8 * i) >> 28), (float)(v << (24 - 8 * i) >> 28));
   return __builtin_bit_cast(bf8_t, p);
+}
+
+// One output by fp32 FMAs, where out_of_terms(v) says that the terms may not
+// have held it.  Past fp32's range (an infinite or NaN activation, or finite
+// ones whose unit's sum overflows before its gain) the gain goes in first; below,
+// last, as a unit's sum of subnormal activations is exact.  A NaN stays one, so
+// it ends the row.  The check of a tile's outputs is within the runs' noise (6144
+// x 1536 at 37 lanes 13.1 us, 13.1 without); one output's bits each, gathered as
+// it is stored, cost 0.5 us.
+__device__ __forceinline__ float few_dot(const float *x, const uint8_t *codes, const float *gains,
+                                         int group_shift, int units, float v) {
+  const bool below = fabsf(v) < 1.0f;
+  float sum = 0.0f;
+  for (int u = 0; u < units && sum == sum; ++u) {
+    const float gain = gains[u >> group_shift];
+    const float first = below ? 1.0f : gain, last = below ? gain : 1.0f;
+    const uint4_t c = *reinterpret_cast<const uint4_t *>(codes + 16 * u);
+    float dot = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float4_t a = *reinterpret_cast<const float4_t *>(x + 32 * u + 4 * i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int code = (int)((c[i / 2] >> (16 * (i & 1) + 4 * e)) & 15u) - 8;
+        dot = __builtin_fmaf((float)code * first, a[e], dot);
+      }
+    }
+    sum = __builtin_fmaf(last, dot, sum);
+  }
+  return sum;
 }
 
 template <int WN, int WM, int KS, int NB, int MB, int STAGES>
@@ -262,9 +293,38 @@ __global__ __launch_bounds__(64 * WN * WM * KS, WN * WM * KS <= 4 ? 2 : WN * WM 
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
         const int nn = n0 + (wn * NB + j) * 16 + n;
-        if (nn < g.N) g.out[(size_t)m * (size_t)g.out_stride + nn] = acc[i][j][r];
+        if (nn >= g.N) continue;
+        g.out[(size_t)m * (size_t)g.out_stride + nn] = acc[i][j][r];
       }
     }
+  uint32_t worst = 0;
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) worst = max(worst, term_range(acc[i][j][r]));
+  if (worst <= kTermRange) return;
+  // Some to form again, one by one.
+  uint32_t again = 0;
+  static_assert(MB * NB * 4 <= 32, "a bit an output");
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+        if (m0 + (wm * MB + i) * 16 + 4 * gq + r < g.M && n0 + (wn * NB + j) * 16 + n < g.N &&
+            out_of_terms(acc[i][j][r]))
+          again |= 1u << ((i * NB + j) * 4 + r);
+  for (; again; again &= again - 1) {
+    const int bit = __builtin_ctz(again), tile = bit / 4;
+    const int m = m0 + (wm * MB + tile / NB) * 16 + 4 * gq + bit % 4;
+    const int nn = n0 + (wn * NB + tile % NB) * 16 + n;
+    float *out = g.out + (size_t)m * (size_t)g.out_stride + nn;
+    *out = few_dot(g.act + (size_t)m * (size_t)g.act_stride, g.codes + (size_t)nn * (size_t)g.row_stride,
+                   g.gains + (size_t)nn * (size_t)g.gain_stride, g.group_shift, units, *out);
+  }
 }
 
 // ---- forms and their choice -----------------------------------------------

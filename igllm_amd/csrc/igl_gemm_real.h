@@ -108,6 +108,17 @@ __device__ __forceinline__ void split3(const float4_t lo, const float4_t hi, bf8
   t[2] = __builtin_bit_cast(bf8_t, p2);
 }
 
+// Whether an output may be off because its activations' terms left their
+// range: infinite or NaN, or so small (below 2^-90, but not zero) that what three
+// bf16 terms cut off an activation, less than their last bit 2^-133 of it, could
+// count.  An output of activations all below 2^-133 comes out zero.
+// term_range is past kTermRange for all of these, and for zero.
+constexpr uint32_t kTermLeast = (127u - 90u) << 24, kTermRange = 0xFEFFFFFFu - kTermLeast;
+
+__device__ __forceinline__ uint32_t term_range(float v) { return (__float_as_uint(v) << 1) - kTermLeast; }
+
+__device__ __forceinline__ bool out_of_terms(float v) { return v != 0.0f && term_range(v) > kTermRange; }
+
 // Eight weights as their bf16 terms: one (bf16), or two (binary16).
 template <bool HALF>
 __device__ __forceinline__ void weight_terms(const uint4_t w, bf8_t (&t)[HALF ? 2 : 1]) {

@@ -47,3 +47,42 @@ def test_few_lanes(backend, N, K, lanes, group, spread):
     x = act[:, :K].astype(np.float64)
     bound = (12 + 2 + 7 + K / 2048 + 15) * 2.0 ** -24 * (np.abs(x) @ np.abs(value).T)
     assert np.all(np.abs(got - x @ value.T) <= bound)
+
+
+# K split sixteen and eight ways, more than one wave row
+@pytest.mark.parametrize("N,K,lanes", [(300, 512, 12), (4100, 544, 40), (12300, 96, 60)])
+def test_few_lanes_activation_range(backend, N, K, lanes):
+    """Lanes of activations near fp32's ends: unit sums past its range that
+    their gains bring back, values below the three terms' last bit, subnormal
+    ones, zero, infinite and NaN.  Formed again, an output passes its unit's 32
+    additions and one a unit, a weight's rounding, and where it is subnormal
+    half of 2^-149 a unit."""
+    rng = np.random.default_rng(N)
+    codes = rng.integers(0, 256, size=(N, K // 2), dtype=np.uint8)
+    gains = np.abs(rng.normal(0, 0.02, size=(N, K // 32))).astype(np.float32)
+    act = rng.normal(size=(lanes, K)).astype(np.float32)
+    for lane, scale in ((1, 2.0 ** 123), (2, 2.0 ** -112), (3, 2.0 ** -119), (4, 2.0 ** -128), (5, 0.0)):
+        act[lane] *= np.float32(scale)
+    act[6, 3], act[7, K - 1], act[8, 40] = np.inf, -np.inf, np.nan
+    cp = backend.attach(make_plane(codes, gains, K))
+    dev_act, dev_out = backend.upload(act), backend.alloc(lanes * N * 4)
+    backend.gemv_dev(cp, dev_act, K, lanes, dev_out, N)
+    backend.sync()
+    got = dev_out.get(np.float32, lanes * N).reshape(lanes, N)
+    dev_act.free()
+    dev_out.free()
+    backend.detach(cp)
+    value = np.empty((N, K), np.float64)
+    value[:, 0::2] = (codes & 15).astype(np.float64) - 8
+    value[:, 1::2] = (codes >> 4).astype(np.float64) - 8
+    value *= np.repeat(gains.astype(np.float64), 32, axis=1)
+    x = act.astype(np.float64)
+    finite = [m for m in range(lanes) if m not in (6, 7, 8)]
+    want = x[finite] @ value.T
+    assert np.abs(want).max() < 3.4e38
+    bound = (32 + 1 + K / 32 + 2) * 2.0 ** -24 * (np.abs(x[finite]) @ np.abs(value).T) + K / 32 * 2.0 ** -150
+    assert np.all(np.abs(got[finite] - want) <= bound)
+    for m, k in ((6, 3), (7, K - 1)):
+        side = np.sign(value[:, k]) * np.sign(act[m, k])
+        assert np.array_equal(got[m], np.where(side == 0, np.nan, side * np.inf).astype(np.float32), equal_nan=True)
+    assert np.isnan(got[8]).all()
