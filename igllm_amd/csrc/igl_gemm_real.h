@@ -11,9 +11,11 @@
 // left (8 + 8 + 8 significand bits, no rounding, bf16's exponent range is
 // fp32's); a bf16 weight is one term and a binary16 weight two (8 + 3 bits).
 // A product of two terms is exact in fp32, and v_mfma_f32_16x16x32_bf16 adds
-// it into an fp32 accumulator.  An output that comes out NaN (an infinite or
-// NaN value among its operands: a zero term against an infinity) is formed
-// again by plain fp32 FMAs over the row, which is what gemv_real_kernel gives.
+// it into an fp32 accumulator.  An output that comes out infinite or NaN (an
+// infinite or NaN value among its operands: a zero term against an infinity), or
+// so small that the terms may have cut its activations off (out_of_terms), is
+// formed again by plain fp32 FMAs over the row, which is what gemv_real_kernel
+// gives.
 //
 // Rounding.  One accumulator over all of K measured 4.2e-7 off the 64-bit
 // product at K = 1536 (N(0,1) activations, 2-norm): the matrix core rounds
@@ -140,7 +142,7 @@ __device__ __forceinline__ void weight_terms(const uint4_t w, bf8_t (&t)[HALF ? 
 
 // One output by fp32 FMAs over the row; a NaN stays one, so it ends the row.
 template <bool HALF>
-__device__ __attribute__((noinline)) float plain_dot(const float *x, const uint16_t *w, int K) {
+__device__ __forceinline__ float plain_dot(const float *x, const uint16_t *w, int K) {
   float sum = 0.0f;
   for (int k = 0; k < K && sum == sum; ++k) {
     const float v = HALF ? (float)__builtin_bit_cast(_Float16, w[k]) : __uint_as_float((uint32_t)w[k] << 16);
@@ -343,11 +345,36 @@ __global__ __launch_bounds__(64 * WN * WM * KS, WN * WM * KS <= 4 ? 2 : WN * WM 
       for (int j = 0; j < NB; ++j) {
         const int nn = n0 + (wn * NB + j) * 16 + n;
         if (nn >= g.N) continue;
-        float v = acc[i][j][r];
-        if (v != v) v = plain_dot<HALF>(g.act + (size_t)m * (size_t)g.act_stride, g.rows + (size_t)nn * (size_t)g.K, g.K);
-        g.out[(size_t)m * (size_t)g.out_stride + nn] = v;
+        g.out[(size_t)m * (size_t)g.out_stride + nn] = acc[i][j][r];
       }
     }
+  uint32_t worst = 0;
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) worst = max(worst, term_range(acc[i][j][r]));
+  if (worst <= kTermRange) return;
+  // Some to form again, one by one.
+  uint32_t again = 0;
+  static_assert(MB * NB * 4 <= 32, "a bit an output");
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+        if (m0 + (wm * MB + i) * 16 + 4 * gq + r < g.M && n0 + (wn * NB + j) * 16 + n < g.N &&
+            out_of_terms(acc[i][j][r]))
+          again |= 1u << ((i * NB + j) * 4 + r);
+  for (; again; again &= again - 1) {
+    const int bit = __builtin_ctz(again), tile = bit / 4;
+    const int m = m0 + (wm * MB + tile / NB) * 16 + 4 * gq + bit % 4;
+    const int nn = n0 + (wn * NB + tile % NB) * 16 + n;
+    g.out[(size_t)m * (size_t)g.out_stride + nn] =
+        plain_dot<HALF>(g.act + (size_t)m * (size_t)g.act_stride, g.rows + (size_t)nn * (size_t)g.K, g.K);
+  }
 }
 
 // ---- forms and their choice -----------------------------------------------

@@ -85,3 +85,20 @@ def test_real_product_of_infinities(backend, kind):
     keep = [n for n in range(N) if n != 9]
     assert np.array_equal(got[rest, 9], np.float32(np.sign(x[rest, 40]) * np.inf))
     assert np.allclose(got[np.ix_(rest, keep)], want[np.ix_(rest, keep)], rtol=0, atol=1e-5)
+
+
+# K split eight and four ways, and not
+@pytest.mark.parametrize("kind", ["bf16", "f16"])
+@pytest.mark.parametrize("N,K,lanes", [(300, 512, 12), (8960, 544, 48), (2560, 96, 512)])
+def test_real_product_of_small_activations(backend, kind, N, K, lanes):
+    """Lanes of activations near the three terms' last bit (2^-133) and below,
+    where an output is formed again by FMAs: K additions at most, and half of
+    2^-149 each where they are subnormal."""
+    act, rows, value, stride = case(kind, N, K, lanes, 5)
+    for lane, scale in ((1, 2.0 ** -112), (2, 2.0 ** -119), (3, 2.0 ** -128), (4, 0.0)):
+        act[lane] *= np.float32(scale)
+    got = product(backend, kind, N, K, lanes, act, rows, stride)
+    x = act[:, :K].astype(np.float64)
+    bound = (K + 2) * (2.0 ** -24 * (np.abs(x) @ np.abs(value).T) + 2.0 ** -150)
+    bound[5:] = (16 + K / 128 + 15 + 2) * 2.0 ** -24 * (np.abs(x[5:]) @ np.abs(value).T)
+    assert np.all(np.abs(got - x @ value.T) <= bound)
