@@ -357,8 +357,13 @@ static int level_step_k(int bits) { return bits == 8 ? 64 : 128; }
 // A launch takes 64 x 64 tiles (lanes x rows) while three workgroups a CU hold
 // them all (768), else 64 x 128 (to 768 tiles, 1536 for 2- and 4-bit codes), else
 // 128 x 128 (to 1024), else 256 x 192.  Many small workgroups a CU hide each
-// other's stages and closes; the widest tile reads the least.  us, the former
-// 256 x 256 tile (K in slices) -> the choice, its neighbours:
+// other's stages and closes; the widest tile reads the least.  From 32 steps on
+// (K = 4096, 2048 for 8-bit codes) the stages outweigh the close and wider tiles
+// come sooner for 4- and 8-bit codes (kLevelLong): with the limits above 10416 x
+// 7296 8-bit at 528 lanes took 112 us (64 x 128) where the former tile took 91 and
+// 128 x 128 takes 87, 11360 x 4736 4-bit at 988 lanes 96 where it took 84 and 128 x
+// 128 takes 84.  us, the former 256 x 256 tile (K in slices) -> the choice, its
+// neighbours:
 //   6144 x 1536, 4-bit:  64 lanes 16.0 -> 11.0, 500 lanes 38.7 -> 16.7 (64 x 128
 //     17.4), 1000 lanes 47.9 -> 22.6 (64 x 64 26.5, 128 x 128 24.5), 2047 lanes 44.8
 //     -> 38.7 (128 x 128 39.9)
@@ -372,9 +377,13 @@ static int level_step_k(int bits) { return bits == 8 ? 64 : 128; }
 // and more (their int32 partials and the close cost a launch): 1536 x 6144 at 64
 // lanes 22.1 unsplit, 14.1 in slices; 6144 x 1536 (twelve steps) 11.0 unsplit, 12.2.
 struct LevelShape {
-  int mt, nt, tiles, tiles_8bit;
+  int mt, nt;
 };
-constexpr LevelShape kLevelForms[] = {{2, 1, 768, 768}, {2, 2, 1536, 768}, {4, 2, 1024, 1024}, {8, 3, 0, 0}};
+constexpr LevelShape kLevelForms[] = {{2, 1}, {2, 2}, {4, 2}, {8, 3}};
+// the most tiles of a form that a launch takes, 2-, 4- and 8-bit codes
+constexpr int kLevelTiles[3][3] = {{768, 768, 768}, {1536, 1536, 768}, {1024, 1024, 1024}};
+constexpr int kLevelLong[3][3] = {{768, 512, 256}, {1536, 512, 256}, {1024, 1024, 512}};
+constexpr int kLevelLongSteps = 32;
 
 struct LevelPlan {
   int form, slices;
@@ -385,7 +394,7 @@ static LevelPlan level_plan(int M, int N, int K, int bits) {
   for (int form = 0;; ++form) {
     const LevelShape &f = kLevelForms[form];
     const long tiles = (long)((M + 32 * f.mt - 1) / (32 * f.mt)) * ((N + 64 * f.nt - 1) / (64 * f.nt));
-    if (form < 3 && tiles > (bits == 8 ? f.tiles_8bit : f.tiles)) continue;
+    if (form < 3 && tiles > (steps < kLevelLongSteps ? kLevelTiles : kLevelLong)[form][bits / 4]) continue;
     int slices = 1;
     while (slices < 16 && tiles * slices < 128 && steps % (2 * slices) == 0 && steps / (2 * slices) >= 8) slices *= 2;
     return LevelPlan{form, slices};
@@ -404,6 +413,8 @@ extern "C" int igl_gemm_level_fits(int bits, int code_bias, int K) {
   if (code_bias != (1 << (bits - 1))) return 0;
   return K >= level_step_k(bits) && K % level_step_k(bits) == 0;
 }
+
+extern "C" int igl_gemm_level_form(int M, int N, int K, int bits) { return level_plan(M, N, K, bits).form; }
 
 extern "C" size_t igl_gemm_level_work_bytes(int M, int N, int K, int bits) {
   const int slices = level_plan(M, N, K, bits).slices;

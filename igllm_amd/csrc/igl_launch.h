@@ -284,8 +284,10 @@ hipError_t igl_launch_fill(float *dst, size_t n, float value, hipStream_t stream
  * NaN gives NaN outputs.  Fits: 2-, 4- or 8-bit codes with code_bias
  * 2^(bits-1), K a multiple of 128 (64 for 8-bit); row_stride a multiple of 16;
  * act 16-byte aligned with act_stride % 4 == 0.  `work` holds
- * igl_gemm_level_work_bytes(M, N, K, bits) bytes. */
+ * igl_gemm_level_work_bytes(M, N, K, bits) bytes.  form: the tile a launch
+ * takes, 0-3 (64 x 64, 64 x 128, 128 x 128, 256 x 192; for tests). */
 int igl_gemm_level_fits(int bits, int code_bias, int K);
+int igl_gemm_level_form(int M, int N, int K, int bits);
 size_t igl_gemm_level_work_bytes(int M, int N, int K, int bits);
 hipError_t igl_launch_gemm_level(const float *act, int act_stride, const uint8_t *codes, long long row_stride,
                                  int bits, int code_flip, int code_bias, const igl_gemm_close *close, float *out,

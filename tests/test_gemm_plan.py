@@ -93,3 +93,15 @@ def test_bench_shapes(lib):
             (1024, 2048, 8192): (2, 1), (2048, 2048, 8192): (1, 1)}
     for (M, N, K), plan in want.items():
         assert (lib.igl_gemm_form(M, N, K, 1), lib.igl_gemm_slices(M, N, K, 1)) == plan, (M, N, K)
+
+
+# 64 x 64, 64 x 128, 128 x 128, 256 x 192 (lanes x rows)
+@pytest.mark.parametrize("M,N,K,bits,form", [
+    (500, 6144, 1536, 4, 0), (1000, 6144, 1536, 4, 1), (2047, 6144, 1536, 4, 1), (2047, 12288, 1536, 4, 3),
+    (1000, 8192, 1920, 8, 2), (500, 6144, 1920, 8, 0),
+    # long rows leave the small tiles sooner: where they did not, slower than one 256 x 256 tile
+    (528, 10416, 7296, 8, 2), (386, 11200, 7040, 8, 2), (333, 7104, 4736, 8, 2), (988, 11360, 4736, 4, 2),
+    (2046, 3680, 5632, 4, 2), (528, 10416, 7296, 2, 1), (63, 96, 6144, 4, 0),
+])
+def test_level_tiles(lib, M, N, K, bits, form):
+    assert lib.igl_gemm_level_form(M, N, K, bits) == form
