@@ -344,9 +344,9 @@ static hipError_t few_launch(const GemmFewArgs &a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// The tiles (weight rows x lanes, K split eight or sixteen ways inside the
-// workgroup) in the order a launch tries them; it takes the first whose grid
-// its rounds hold.  Replayed, us, the chosen form against its neighbours:
+// The tiles (weight rows x lanes, K split sixteen ways inside the workgroup in
+// the first two, eight in the others, four in 64 x 64) in the order a launch
+// tries them; it takes the first whose grid its rounds hold.  Replayed, us, the chosen form against its neighbours:
 //   6144 x 1536: 24 lanes 48 x 16 8.1 (32 x 32 10.0, 64 x 32 13.9), 37 lanes 32 x
 //                48 12.6 (64 x 32 14.6), 63 lanes 48 x 16 11.6 (64 x 32 14.7)
 //   1536 x 6144: 24 lanes 16 x 16 13.8 (32 x 16 17.9), 63 lanes 32 x 16 18.4 (16 x
@@ -383,6 +383,8 @@ extern "C" int igl_gemm_few_fits(int lanes, int N, int K) {
   return N >= 1 && K >= 32 && K % 32 == 0 && lanes <= 63 &&
          (lanes >= 17 || (lanes >= 9 && (K < 4096 || N >= 4096)));
 }
+
+extern "C" int igl_gemm_few_form(int lanes, int N) { return few_form(lanes, N); }
 
 // Arguments as igl_launch_gemv_q4's (code bias 8), activations 16-byte aligned
 // with act_stride % 4 == 0, no workspace.

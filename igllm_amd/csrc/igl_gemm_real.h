@@ -446,6 +446,8 @@ extern "C" int igl_gemm_real_fits(int real_type, int lanes, int N, int K) {
          K % 32 == 0;
 }
 
+extern "C" int igl_gemm_real_form(int lanes, int N) { return real_form(lanes, N); }
+
 extern "C" hipError_t igl_launch_gemm_real(const void *rows, int real_type, const float *act, int act_stride,
                                            int lanes, float *out, int out_stride, int N, int K, hipStream_t stream) {
   if (!igl_gemm_real_fits(real_type, lanes, N, K) || (((uintptr_t)act) & 15u) || (((uintptr_t)rows) & 15u) ||

@@ -79,13 +79,15 @@ hipError_t igl_launch_gemv_real(const void *rows, int real_type, const float *ac
 
 /* The same product on the bf16 matrix cores (bf16 and binary16 rows, five
  * lanes and more, K a multiple of 32; arguments as igl_launch_gemv_real's,
- * no workspace). */
+ * no workspace).  form: the tile a launch takes, 0-6 (for tests). */
+int igl_gemm_real_form(int lanes, int N);
 int igl_gemm_real_fits(int real_type, int lanes, int N, int K);
 hipError_t igl_launch_gemm_real(const void *rows, int real_type, const float *act, int act_stride,
                                 int lanes, float *out, int out_stride, int N, int K, hipStream_t stream);
 
 /* A 4-bit plane (code bias 8, no zero points) times 9 to 63 lanes on the bf16
- * matrix cores; no workspace. */
+ * matrix cores; no workspace.  form: the tile a launch takes, 0-7 (for tests). */
+int igl_gemm_few_form(int lanes, int N);
 int igl_gemm_few_fits(int lanes, int N, int K);
 hipError_t igl_launch_gemm_few(const uint8_t *codes, long long row_stride, const float *gains,
                                int gain_stride, int group_shift, const float *act, int act_stride,

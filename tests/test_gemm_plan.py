@@ -105,3 +105,25 @@ def test_bench_shapes(lib):
 ])
 def test_level_tiles(lib, M, N, K, bits, form):
     assert lib.igl_gemm_level_form(M, N, K, bits) == form
+
+
+def test_gpu_cases_take_every_tile(lib):
+    """The parametrised GPU tests of the few-lane, real and integer products
+    launch each of their tiles, and each with more steps of K than it has
+    stages (the ring refilled)."""
+    import test_gpu_gemm_few as few
+    import test_gpu_gemm_level as level
+    import test_gpu_gemm_real as real
+
+    # units of K a step (the K split), and stages, of each tile
+    few_steps = [(16, 2), (16, 3), (8, 3), (8, 3), (8, 2), (8, 3), (8, 3), (4, 3)]
+    seen = {lib.igl_gemm_few_form(lanes, N) for N, K, lanes, _ in few.CASES
+            if K // 32 > few_steps[lib.igl_gemm_few_form(lanes, N)][0] * few_steps[lib.igl_gemm_few_form(lanes, N)][1]}
+    assert seen == set(range(8))
+    real_steps = [(8, 3), (8, 3), (4, 4), (8, 2), (8, 2), (4, 3), (1, 4)]
+    seen = {lib.igl_gemm_real_form(lanes, N) for N, K, lanes in real.CASES
+            if K // 32 > real_steps[lib.igl_gemm_real_form(lanes, N)][0] * real_steps[lib.igl_gemm_real_form(lanes, N)][1]}
+    assert seen == set(range(7)), seen
+    for bits in (2, 4, 8):
+        step = 64 if bits == 8 else 128
+        assert {lib.igl_gemm_level_form(lanes, N, K, bits) for N, K, lanes in level.CASES if K // step > 3} == set(range(4))

@@ -1,11 +1,10 @@
 """GPU parity of the wide attention launch (igl_launch_attend with 64 lanes or
-more, a prefill pass): one workgroup a lane and key/value head walks the
-lane's chunks and merges them online, instead of a workgroup a chunk and a
-fold launch.
+more, a prefill pass): tiles of lanes walk their chunks and merge them online,
+instead of a workgroup a chunk and lane and a fold launch.
 
 For lanes at positions p .. p + lanes - 1 over a byte ring (e4m3 or int8),
 each lane seeing the positions up to its own inside its window:
-- every lane's blend against the same lanes launched 63 at a time (the chunk
+- every lane's blend against the same lanes launched alone (always the chunk
   workgroups and their fold): the two forms add the same terms in another
   order, bar 1e-5 max|o| + 1e-7;
 - sampled lanes against the oracle (oracle_attend over the lane's span), bar
@@ -21,7 +20,6 @@ import oracle_lib as ol
 pytestmark = pytest.mark.gpu
 
 HEADS = 8
-NARROW = 63  # lanes a launch below the wide form takes
 
 
 def _bind(lib):
@@ -70,20 +68,19 @@ def test_wide_attention(backend, lanes, window, place0, head, fmt, kv_count, pad
     narrow = backend.alloc(lanes * q_stride * 4)
     for b in (wide, narrow):  # the pad columns compare equal
         b.put(np.zeros(lanes * q_stride, np.float32))
-    work_floats = max([lib.igl_attend_work_floats(place0 + at, window, min(NARROW, lanes - at), kv_count * HEADS,
-                                                  head) for at in range(0, lanes, NARROW)] + [1])
+    work_floats = max([lib.igl_attend_work_floats(place0, window, lanes, kv_count * HEADS, head)] +
+                      [lib.igl_attend_work_floats(place0 + at, window, 1, kv_count * HEADS, head) for at in range(lanes)])
     work = backend.alloc(work_floats * 4)
     try:
         rc = fn(dk.ptr, dv.ptr, fmt, scale, scale, cache_span, kv_width, kv_count, HEADS, head, dq.ptr, q_stride,
                 place0, None, window, lanes, score_scale, wide.ptr, work.ptr, stream)
         assert rc == 0
-        for at in range(0, lanes, NARROW):
-            n = min(NARROW, lanes - at)
+        backend.sync()
+        for at in range(lanes):  # on one stream: each launch's partials are folded before the next writes
             rc = fn(dk.ptr, dv.ptr, fmt, scale, scale, cache_span, kv_width, kv_count, HEADS, head,
-                    dq.ptr + at * q_stride * 4, q_stride, place0 + at, None, window, n, score_scale,
+                    dq.ptr + at * q_stride * 4, q_stride, place0 + at, None, window, 1, score_scale,
                     narrow.ptr + at * q_stride * 4, work.ptr, stream)
             assert rc == 0
-            backend.sync()  # the next group reuses the partials
         backend.sync()
         got = wide.get(np.float32, lanes * q_stride).reshape(lanes, q_stride)
         ref = narrow.get(np.float32, lanes * q_stride).reshape(lanes, q_stride)

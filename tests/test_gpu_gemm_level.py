@@ -16,11 +16,15 @@ from igllm_amd.backend import Backend, make_plane
 pytestmark = pytest.mark.gpu
 
 
-# each tile's edges (64 x 64, 64 x 128, 128 x 128, 256 x 192: lanes x rows), K
+# each tile's edges (64 x 64, 64 x 128, 128 x 128, 256 x 192: lanes x rows; in
+# every width all four, with more steps than the stages: test_gemm_plan), K
 # slices, one step, lanes below and past the GEMM's former floor
+CASES = [(16, 128, 5), (300, 2048, 63), (96, 6144, 64), (1000, 256, 65), (4112, 384, 767), (6160, 128, 1030),
+         (12304, 128, 1990), (4100, 640, 1000), (8100, 640, 2000), (12304, 640, 1990)]
+
+
 @pytest.mark.parametrize("bits", [2, 4, 8])
-@pytest.mark.parametrize("N,K,lanes", [(16, 128, 5), (300, 2048, 63), (96, 6144, 64), (1000, 256, 65), (4112, 384, 767),
-                                       (6160, 128, 1030), (12304, 128, 1990)])
+@pytest.mark.parametrize("N,K,lanes", CASES)
 def test_lanes_equal_single_lanes(backend, bits, N, K, lanes):
     rng = np.random.default_rng(N + K + lanes + bits)
     codes = rng.integers(0, 256, size=(N, (K * bits // 8 + 15) // 16 * 16), dtype=np.uint8)

@@ -49,11 +49,15 @@ def case(kind, N, K, lanes, seed, spread=False):
 
 
 # every tile form's edges: 16 x 16, 32 x 16 (one and two a CU), 32 x 32, 64 x
-# 32, 64 x 64 split and unsplit; K of one step, and not a whole K split
+# 32, 64 x 64 split and unsplit (test_gemm_plan checks that all are seen); K of
+# one step, and not a whole K split
+CASES = [(1, 32, 5), (17, 96, 17), (300, 288, 15), (4100, 352, 16), (8193, 64, 13), (4097, 160, 33), (8190, 96, 31),
+         (4090, 544, 65), (8960, 1536, 70), (16, 2048, 500), (4100, 1056, 16), (8193, 1568, 13), (8190, 1056, 31),
+         (8960, 1536, 64), (8950, 544, 48)]
+
+
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
-@pytest.mark.parametrize("N,K,lanes", [(1, 32, 5), (17, 96, 17), (300, 288, 15), (4100, 352, 16), (8193, 64, 13),
-                                       (4097, 160, 33), (8190, 96, 31), (4090, 544, 65), (8960, 1536, 70),
-                                       (16, 2048, 500)])
+@pytest.mark.parametrize("N,K,lanes", CASES)
 @pytest.mark.parametrize("spread", [False, True])
 def test_real_product(backend, kind, N, K, lanes, spread):
     act, rows, value, stride = case(kind, N, K, lanes, N + K + lanes, spread)
@@ -63,15 +67,19 @@ def test_real_product(backend, kind, N, K, lanes, spread):
     assert np.all(np.abs(got - x @ value.T) <= bound)
 
 
+# 16 x 16 and 64 x 64, K split eight and four ways, and 64 x 64 unsplit
+@pytest.mark.parametrize("N,lanes", [(70, 20), (8960, 48), (4100, 500)])
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
-def test_real_product_of_infinities(backend, kind):
+def test_real_product_of_infinities(backend, kind, N, lanes):
     """An infinite or NaN operand gives what the FMAs of a row give, and
-    leaves the other outputs alone."""
-    N, K, lanes = 70, 256, 20
+    leaves the other outputs alone; the largest finite activations have three
+    finite terms."""
+    K = 256
     act, rows, value, stride = case(kind, N, K, lanes, 3)
     want = act[:, :K].astype(np.float64) @ value.T
     act[2, 5], act[7, 100], act[11, 255] = np.inf, -np.inf, np.nan
-    act[13, :K] = np.float32(3.4e38)  # every term finite
+    act[13, :K] = 0.0
+    act[13, 17] = np.float32(3.4e38)
     rows[9, 40] = 0x7F80 if kind == "bf16" else np.float16(np.inf)
     value = ((rows.astype(np.uint32) << 16).view(np.float32) if kind == "bf16" else rows).astype(np.float64)
     got = product(backend, kind, N, K, lanes, act, rows, stride)
@@ -81,6 +89,9 @@ def test_real_product_of_infinities(backend, kind):
             full = x[m] * value[n]
             total = np.nan if np.isnan(full).any() else full.sum()
             assert np.array_equal(got[m, n], np.float32(total), equal_nan=True), (m, n)
+    big = np.float64(act[13, 17]) * value[:, 17]
+    big[9] = np.nan  # 0 x inf
+    assert np.allclose(got[13], big, rtol=2.0 ** -22, atol=0, equal_nan=True)
     rest = [m for m in range(lanes) if m not in (2, 7, 11, 13)]
     keep = [n for n in range(N) if n != 9]
     assert np.array_equal(got[rest, 9], np.float32(np.sign(x[rest, 40]) * np.inf))
