@@ -23,7 +23,11 @@
 #define IGL_GEMM_FLOOR 64 /* lanes from which mat_mat takes the MFMA GEMM */
 /* lanes from which a calibrated plane takes the integer GEMM: the level GEMV
  * forms each lane's sums apart (6144 x 1536, 8 lanes 23 us, 63 lanes 178; the
- * GEMM 11) */
+ * GEMM 10 and 11).  Five is not the crossing everywhere: of the planes of an E2B
+ * layer three and four lanes take as long on the GEMV as five on the GEMM or
+ * longer (6144 x 1536 11.2 and 12.4 us against 9.6, 1536 x 6144 12.6 and 15.7
+ * against 12.5), and on the smallest planes five are slower on the GEMM (272 x
+ * 1408 8-bit 8.8 -> 9.7). */
 #define IGL_LEVEL_FLOOR 5
 
 struct igl_device_plane {

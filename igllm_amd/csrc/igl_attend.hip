@@ -671,10 +671,9 @@ __global__ __launch_bounds__(256) void attend_split_kernel(AttendArgs a) {
 // 32 rows, 2000 of them products on each SIMD).  At 2047 lanes, us, against one
 // workgroup a lane: 2048 positions of 512-dim heads 450 -> 101 (69 GFLOP of
 // products, two terms each: 680 TFLOP/s), a 512 window of 256-dim heads 104 -> 34;
-// 511 lanes 57 -> 22.  Against an earlier form at 118 us: four waves of 128 dims,
-// two workgroups a CU, 129 (a chunk's chain is 8800 cycles, and the longest
-// tile's chunks bound the launch); the keys in registers instead of LDS spilled
-// (166).
+// 511 lanes 57 -> 22.  Slower: four waves of 128 dims, two workgroups a CU (9%: a
+// chunk's chain is 8800 cycles, and the longest tile's chunks bound the launch);
+// the keys in registers instead of LDS (41%: spills).
 //
 // Per chunk: scores S = q_lo . K^T + q_hi . K^T (the waves' sums added in wave
 // order), probabilities p = e^(S - base) to LDS as two binary16 terms, and total
@@ -1167,8 +1166,9 @@ static int attend_blocks(int place0, int window, int lanes) {
 //     lanes at 16000 26.7 -> 14.9, but 4 lanes of the window 7.7 against 7.9, 16
 //     lanes 8.5 against 8.9, 2 lanes at 16000 (502 chunk workgroups) 12.8
 //     against 13.2.
-// Tiles of two lanes up to 512 of them, of four beyond (1000 lanes of 512 dims
-// 43.2 us in twos, 49.3 in fours; 2047 lanes 153 against 118).
+// Tiles of two lanes up to 512 of them, of four beyond (us in twos and in fours:
+// 1000 lanes of 512 dims 46.9, 49.9; 1100 54.4, 55.4; 1500 82.0, 72.3; 2047 127.8,
+// 101.5; 2047 of a 512 window of 256 dims 41.0, 36.7).
 //
 // Few tiles are cut into segments of their chunks, folded by a second launch:
 // as many as fill 256 workgroups, 512 (512 dims) or 1024 (256 dims) where a

@@ -660,7 +660,10 @@ constexpr FormShape kFormsLo[] = {
 // so the widest form that fills the CUs is often not it: 6144 x 1536 at 1000
 // lanes, fp32, 384 tiles of 128 x 128 are two rounds, 79.9 us, 1536 of 64 x 64
 // three, 69.9; 12288 x 1536 at 1000 lanes 120 (form 0) -> 107 (128 x 128); 6144 x
-// 1536 at 2047 lanes 123 -> 110.
+// 1536 at 2047 lanes 123 -> 110.  The costs are K = 1536's; over 170 random shapes
+// (256-12288 rows, K 256-8192, 64-2047 lanes) the choice takes 0.99 of the former
+// one's time in the mean, 1.02 at most with one term and 1.03 with two (short
+// rows: the runs' additions below).
 // Against the widest form that filled the CUs (the choice before), replayed,
 // us, bf16 / fp32 activations: 8192 x 2048 at 256 lanes 30.2 / 41.5 -> 27.2 /
 // 35.1 (two a CU); 6144 x 1536 at 128 lanes 22.5 / 30.0 -> 15.0 / 18.7 (64 x 64,

@@ -147,12 +147,18 @@ void igl_plane_detach(igl_desk *desk, igl_plane *sheet);
 
 /* ---- device-resident entries (enqueue on the desk's stream) -------------- */
 
-/* y = W x for `lane_count` lanes of fp32 activations: 1..8 lanes a launch
- * take the HBM-streaming GEMV (more lanes run in chunks of 8); from
- * `igl_gemm_lane_floor()` lanes on, the MFMA GEMM. */
+/* y = W x for `lane_count` lanes of fp32 activations: below
+ * `igl_gemm_lane_floor()` lanes what igl_gemv_dev takes, from there on the MFMA
+ * GEMM (4-bit planes stored value + 8, K a multiple of 64). */
 int igl_mat_mat_dev(igl_desk *desk, const igl_plane *sheet, const float *act_dev, int act_stride,
                     int lane_count, float *out_dev, int out_stride);
-/* Always the GEMV path (lanes in chunks of 8), whatever the lane count. */
+/* Never the prefill GEMM, whatever the lane count: no conversion of the
+ * activations and no workspace but what attaching the plane reserved.  A 4-bit
+ * plane stored value + 8, without zero points, takes the HBM-streaming GEMV to
+ * 8 lanes, the few-lane matrix-core product from 17 to 63 (9 to 16 too, but on
+ * few long rows) where the activations are 16-byte aligned, else the GEMV
+ * sixteen lanes a launch; real planes of bf16 or binary16 rows the matrix cores
+ * from 5 lanes (K a multiple of 32); other kinds the GEMV. */
 int igl_gemv_dev(igl_desk *desk, const igl_plane *sheet, const float *act_dev, int act_stride,
                  int lane_count, float *out_dev, int out_stride);
 /* Batched prefill: bf16 activations [lanes][act_stride] -> bf16 [lanes][out_stride],
