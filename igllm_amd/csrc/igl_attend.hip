@@ -669,25 +669,26 @@ __global__ __launch_bounds__(256) void attend_split_kernel(AttendArgs a) {
 // What bounds it: a chunk's chain between the two barriers (decode, products,
 // the exchanged sums, the exponentials; 6200 cycles a chunk of 512-dim heads at
 // 32 rows, 2000 of them products on each SIMD).  At 2047 lanes, us, against one
-// workgroup a lane: 2048 positions of 512-dim heads 450 -> 101 (69 GFLOP of
-// products, two terms each: 680 TFLOP/s), a 512 window of 256-dim heads 104 -> 34;
+// workgroup a lane: 2048 positions of 512-dim heads 450 -> 99 (69 GFLOP of
+// products, two terms each: 695 TFLOP/s), a 512 window of 256-dim heads 104 -> 34;
 // 511 lanes 57 -> 22.  Slower: four waves of 128 dims, two workgroups a CU (9%: a
 // chunk's chain is 8800 cycles, and the longest tile's chunks bound the launch);
 // the keys in registers instead of LDS (41%: spills).
 //
 // Per chunk: scores S = q_lo . K^T + q_hi . K^T (the waves' sums added in wave
-// order), probabilities p = e^(S - base) to LDS as two binary16 terms, and total
-// and blend = blend e^(old base - base) + (p_lo + p_hi) . V, each chunk's products
-// formed from zero.  A row's base stays while it is at or below the chunk's
-// peak, by ten at most (p below 2^15), else it is the chunk's peak, so p's two
-// terms lose no more than against that peak: half of 2^-24 of the chunk's
-// largest.  Against the running peak, the weights far below an early position's
-// fall under binary16's range: one position 18 above 1000-1900 others, its own
-// value zero, left the blend 12% (256 dims) and 40% (512) off, 4.5% and 8.5%
-// from the chunk that holds it alone, as here.  No base is more than forty under
-// the largest peak, so the scaled sums stay in fp32's range.  It costs 1% of a
-// launch (99.3 -> 100.7 us at 2047 lanes of 512 dims).  Positions a lane does not
-// see have probability zero in its rows.
+// order, in powers of two: log2 e is in the key scale), probabilities p = 2^(S -
+// base) to LDS as two binary16 terms, and total and blend = blend 2^(old base -
+// base) + (p_lo + p_hi) . V, each chunk's products formed from zero.  A row's base
+// is the chunk's peak rounded down, so p's largest is in [1, 2), its two terms
+// lose no more than half of 2^-24 of that, and every scaling is exact.  Against
+// the walk's running peak, the weights far below an early position's fall under
+// binary16's range: one position 18 (base e) above 1000-1900 others, its own value
+// zero, left the blend 12% (256 dims) and 40% (512) off, here 4.4% and 4.9%, the
+// share of the chunk that holds it.  No base is more than 58 under the largest
+// one, so the scaled sums stay in fp32's range.  Off the 64-bit blend at 64-515
+// lanes, scores of deviation 1, 6 and 30: 1.6e-7, 4.5e-7, 9.4e-7 (chunk workgroups
+// 2.2e-7, 7.8e-7, 1.6e-6).  Positions a lane does not see have probability zero in
+// its rows.
 typedef __attribute__((address_space(3))) void attend_lds_t;
 typedef __attribute__((address_space(1))) const void attend_global_t;
 
@@ -769,7 +770,7 @@ __global__ __launch_bounds__(HEAD, 2) void attend_tile_kernel(AttendArgs a) {
   const bool split = gridDim.z > 1;
 
   // the softmax's row of this thread, its lane's visible positions (relative
-  // to start), its largest peak, its base and its running total
+  // to start), its largest base, its base and its running total
   const int row = min(tid / TPR, ROWS - 1);
   const int li = min(row / kAttendGroup, ln - 1);
   const int see_end = pos0 + li - start;  // inclusive
@@ -915,7 +916,7 @@ __global__ __launch_bounds__(HEAD, 2) void attend_tile_kernel(AttendArgs a) {
     // the row's scores of this thread, its peak and total, its probabilities
     if (ROWS * TPR == HEAD || tid < ROWS * TPR) {
       const int p0 = PPT * (tid % TPR);
-      float v[PPT];
+      float raw[PPT], v[PPT];
 #pragma unroll
       for (int e = 0; e < PPT; e += 4) {
         float4_t x[W];
@@ -927,6 +928,7 @@ __global__ __launch_bounds__(HEAD, 2) void attend_tile_kernel(AttendArgs a) {
           for (int w = W / 2; w > 0; w >>= 1)
 #pragma unroll
             for (int j = 0; j < w; ++j) x[j][i] += x[j + w][i];
+          raw[e + i] = x[0][i];
           v[e + i] = x[0][i] * a.key_scale;
         }
       }
@@ -946,15 +948,16 @@ __global__ __launch_bounds__(HEAD, 2) void attend_tile_kernel(AttendArgs a) {
       peak = fmaxf(peak, dpp_move<0x4E>(peak));
       if (TPR >= 8) peak = fmaxf(peak, dpp_move<0x141>(peak));
       if (TPR >= 16) peak = fmaxf(peak, dpp_move<0x140>(peak));
-      top = fmaxf(top, peak);
-      const float over = peak - run_m;
-      const float m = over >= 0.0f && over <= 10.0f ? run_m : fmaxf(peak, top - 40.0f);
-      const float keep = run_m != -INFINITY ? __expf(run_m - m) : 0.0f;
+      const float low = floorf(peak);
+      top = fmaxf(top, low);
+      const float m = fmaxf(low, top - 58.0f);
+      const float keep = run_m != -INFINITY ? __builtin_amdgcn_exp2f(run_m - m) : 0.0f;
       float total = 0.0f;
       _Float16 hi[PPT], lo[PPT];
 #pragma unroll
       for (int e = 0; e < PPT; ++e) {
-        const float p = v[e] != -INFINITY ? __expf(v[e] - m) : 0.0f;
+        // the score's scale and its distance from the base in one rounding
+        const float p = v[e] != -INFINITY ? __builtin_amdgcn_exp2f(__builtin_fmaf(raw[e], a.key_scale, -m)) : 0.0f;
         total += p;
         hi[e] = (_Float16)p;
         lo[e] = (_Float16)(p - (float)hi[e]);
@@ -1052,14 +1055,20 @@ __global__ __launch_bounds__(HEAD, 2) void attend_tile_kernel(AttendArgs a) {
     }
 }
 
+template <bool TWO>
+__device__ __forceinline__ float fold_power(float x) {
+  return TWO ? __builtin_amdgcn_exp2f(x) : __expf(x);
+}
+
 // Folds chunk partials in one memory round trip.  A workgroup per (head, lane,
 // DIMS dims) of 256 threads: thread (d, s) loads, for up to PER chunks
 // c = s, s + 256/DIMS, ..., its dim's partial and the chunk's peak and total
 // together; the slices' peaks meet in LDS (the head's peak M), each thread
 // weights its chunks by e^(peak_c - M), and the slices' sums meet in LDS in a
 // fixed order.  Spans of more chunks than one pass holds take further passes,
-// each rescaled to the running peak.
-template <int DIMS, int PER>
+// each rescaled to the running peak.  TWO: the peaks are powers of two (a tile's
+// segments), not of e.
+template <int DIMS, int PER, bool TWO>
 __global__ __launch_bounds__(256) void attend_fold_kernel(const float *part_out_all,
                                                           const float *part_peak_all,
                                                           const float *part_total_all,
@@ -1106,7 +1115,7 @@ __global__ __launch_bounds__(256) void attend_fold_kernel(const float *part_out_
 #pragma unroll
     for (int i = 0; i < SL; ++i) M = fmaxf(M, red_m[i]);
     if (M != -INFINITY && run_m != -INFINITY && M != run_m) {
-      const float f = __expf(run_m - M);
+      const float f = fold_power<TWO>(run_m - M);
       acc *= f;
       tot *= f;
     }
@@ -1114,7 +1123,7 @@ __global__ __launch_bounds__(256) void attend_fold_kernel(const float *part_out_
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
       const bool in = c0 + sl + SL * u < chunks && m[u] != -INFINITY;
-      const float w = in ? __expf(m[u] - M) : 0.0f;
+      const float w = in ? fold_power<TWO>(m[u] - M) : 0.0f;
       acc += w * v[u];
       tot += w * l[u];
     }
@@ -1303,6 +1312,7 @@ extern "C" hipError_t igl_launch_attend(const uint8_t *key_store, const uint8_t 
   const TilePlan plan = attend_tile_plan(place0, window, lanes, head_count, head_size);
   if (plan.rb) {
     a.final_out = blend_out;
+    a.key_scale = (float)((double)key_scale * unit * score_scale * 1.4426950408889634);  // log2 e
     a.part_peak = work + (size_t)lanes * plan.segments * head_count * head_size;
     a.part_total = a.part_peak + (size_t)lanes * plan.segments * head_count;
     hipError_t e = hipErrorInvalidValue;
@@ -1346,23 +1356,28 @@ static hipError_t attend_fold(const AttendArgs &a, int chunks, int chunk, int pl
   int per = 1;
   while (per < 32 && per * slices < chunks) per *= 2;
   const dim3 fgrid(head_count, lanes, head_size / dims);
-#define IGL_FOLD(D, P)                                                                             \
-  hipLaunchKernelGGL((attend_fold_kernel<D, P>), fgrid, dim3(256), 0, stream, a.part_out,         \
+#define IGL_FOLD(D, P, T)                                                                          \
+  hipLaunchKernelGGL((attend_fold_kernel<D, P, T>), fgrid, dim3(256), 0, stream, a.part_out,      \
                      a.part_peak, a.part_total, chunks, chunk, place0, place_dev, window, extra,   \
                      head_count, head_size, blend_out, q_stride)
-#define IGL_FOLD_PER(D)                                                                            \
+#define IGL_FOLD_PER(D, T)                                                                         \
   switch (per) {                                                                                   \
-    case 1: IGL_FOLD(D, 1); break;                                                                 \
-    case 2: IGL_FOLD(D, 2); break;                                                                 \
-    case 4: IGL_FOLD(D, 4); break;                                                                 \
-    case 8: IGL_FOLD(D, 8); break;                                                                 \
-    case 16: IGL_FOLD(D, 16); break;                                                               \
-    default: IGL_FOLD(D, 32); break;                                                               \
+    case 1: IGL_FOLD(D, 1, T); break;                                                              \
+    case 2: IGL_FOLD(D, 2, T); break;                                                              \
+    case 4: IGL_FOLD(D, 4, T); break;                                                              \
+    case 8: IGL_FOLD(D, 8, T); break;                                                              \
+    case 16: IGL_FOLD(D, 16, T); break;                                                            \
+    default: IGL_FOLD(D, 32, T); break;                                                            \
   }
-  if (dims == 16) {
-    IGL_FOLD_PER(16)
+  const bool two = chunk == 0;  // a tile's segments
+  if (dims == 16 && two) {
+    IGL_FOLD_PER(16, true)
+  } else if (dims == 16) {
+    IGL_FOLD_PER(16, false)
+  } else if (two) {
+    IGL_FOLD_PER(64, true)
   } else {
-    IGL_FOLD_PER(64)
+    IGL_FOLD_PER(64, false)
   }
 #undef IGL_FOLD_PER
 #undef IGL_FOLD
