@@ -78,7 +78,7 @@ struct AttendArgs {
   float key_scale;             // decoded-byte multiplier, score_scale folded in
   float value_scale;
   float *part_out;             // [chunks][head_count][HEAD]
-  float *part_peak;            // [chunks][head_count]
+  float *part_peak;            // [chunks][head_count]; of a tile, log2
   float *part_total;           // [chunks][head_count]
   int head_count;
   // The heads of a decode step or a small block prepared here
